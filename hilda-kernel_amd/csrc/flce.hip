@@ -742,8 +742,8 @@ size_t dx_part_bytes(int64_t C, int64_t Hp, int64_t ldl, int bk, int smax) {
   return best;
 }
 
-// The workspace layout of one candidate (C rows a chunk, the forms, the split cap).
-FlPlan fl_layout(const FlShape& s, int64_t C, bool wt, bool dt, int dw, int smax) {
+// The workspace layout of one candidate (C rows a chunk, the forms, the split cap and its partials' bytes).
+FlPlan fl_layout(const FlShape& s, int64_t C, bool wt, bool dt, int dw, int smax, size_t pb) {
   FlPlan p;
   p.C = C;
   p.nch = s.BT > 0 ? cdiv(s.BT, C) : 0;
@@ -779,11 +779,10 @@ FlPlan fl_layout(const FlShape& s, int64_t C, bool wt, bool dt, int dw, int smax
   if (p.wpad) p.wp = take((size_t)s.V * p.Hp * es);
   if (s.grad) {
     const bool defer = dw == kDwDefer;
-    p.xt = take((size_t)p.Hp * ld_t(defer ? s.BT : C) * es);
+    if (p.dt) p.xt = take((size_t)p.Hp * ld_t(defer ? s.BT : C) * es);
     if (p.wt) p.wtp = take((size_t)p.Hp * p.ldl * es);
     if (p.dt) p.dtp = take((size_t)p.V8 * ld_t(defer ? s.BT : C) * es);
     if (dw == kDwAcc) p.acc = take((size_t)s.V * p.Hp * 4);
-    const size_t pb = dx_part_bytes(C, p.Hp, p.ldl, dx_bk(s.es), smax);
     p.ksplit = pb ? smax : 1;
     p.part = pb ? take(pb) : 0;
   }
@@ -826,14 +825,19 @@ FlPlan vt_layout(const FlShape& s, int64_t Vt, int dw) {
   return p;
 }
 
+// Rate of the 16-bit GEMM kernel in any operand layout, alone on the chip (gemm_wide.h), and of streaming passes
+// over memory. (fp32 plans only compare with each other: the same forms at one rate.)
+constexpr double kGemmRate = 1.4e15, kStreamRate = 5.0e12, kLaunch = 5e-6;
+
 // Modelled time of a vocabulary-tiled candidate: the logits GEMM twice (the
-// log-sum-exp pass, then the gradient pass), the dW GEMM with both operands
-// MN-contiguous, the dX GEMM with W MN-contiguous, idle CUs when a GEMM has
-// fewer than 256 tiles, the row passes' HBM bytes and dX's read-modify-writes.
+// log-sum-exp pass, then the gradient pass), the dW and dX GEMMs, idle CUs when
+// a GEMM has fewer than 256 tiles, the row passes' HBM bytes and dX's
+// read-modify-writes.
 double vt_cost(const FlShape& s, const FlPlan& p) {
-  const double Rg = 1.25e15, Rm = 5.0e12, pen = 1.2, launch = 5e-6;
+  const double Rg = kGemmRate, Rm = kStreamRate, launch = kLaunch;
   const double es = s.es, BT = (double)s.BT, Hp = (double)p.Hp, V = (double)s.V;
-  const double F = 2.0 * BT * Hp * V;
+  // (a 256-row tile costs the same whatever part of it is rows)
+  const double F = 2.0 * (double)(cdiv(s.BT, 256) * 256) * Hp * V;
   // a GEMM of `tiles` 256x256 tiles takes whole waves of 256 (one workgroup a CU)
   auto fill = [](int64_t tiles) {
     tiles = std::max<int64_t>(tiles, 1);
@@ -845,8 +849,7 @@ double vt_cost(const FlShape& s, const FlPlan& p) {
   if (p.wpad) t += 2.0 * es * V * Hp / Rm;
   if (s.grad) {
     t += F / Rg * fill(tb * tv) + 2.0 * BT * V * es / Rm;
-    t += F / Rg * fill(tv * th) * pen * pen;
-    t += F / Rg * fill(tb * th) * pen;
+    t += F / Rg * fill(tv * th) + F / Rg * fill(tb * th);
     const double nt = (double)p.ntiles;
     t += (p.dw == kDwAcc ? 8.0 * BT * Hp * (nt - 1) : 2.0 * es * BT * Hp * (nt - 1)) / Rm;
     t += p.ntiles * 4 * launch;
@@ -854,12 +857,14 @@ double vt_cost(const FlShape& s, const FlPlan& p) {
   return t;
 }
 
-// Modelled time (seconds) of a candidate: GEMMs at a kk-kernel rate, 15% more
-// for a GEMM with an MN-contiguous operand, tile waste of a short chunk, a dX
-// GEMM that leaves CUs idle, and the HBM bytes of the transposes, the dW
-// read-modify-writes, the split partials and the gathers, plus launches.
+// Modelled time (seconds) of a candidate: the GEMMs at one rate whatever their
+// operands' layout, tile waste of a short chunk, a dX GEMM that leaves CUs
+// idle, and the HBM bytes of the transposes, the dW read-modify-writes, the
+// split partials and the gathers, plus launches. (BT 2048, H 4096, V 32000:
+// 1.49 ms with W^T, D^T and X^T, 1.43 without D^T and X^T, 1.40 without W^T, 1.34
+// without any.)
 double fl_cost(const FlShape& s, const FlPlan& p) {
-  const double Rg = 1.25e15, Rm = 5.0e12, pen = 1.2, launch = 5e-6;
+  const double Rg = kGemmRate, Rm = kStreamRate, launch = kLaunch;
   const double es = s.es, BT = (double)s.BT, Hp = (double)p.Hp, V = (double)s.V;
   const double F = 2.0 * BT * Hp * V;
   // row waste of a chunk's last 256-row tile, and whole waves of 256 workgroups (one a CU)
@@ -875,16 +880,16 @@ double fl_cost(const FlShape& s, const FlPlan& p) {
   if (s.grad) {
     const int64_t tiles = cdiv(p.C, 256) * cdiv(p.Hp, 256);
     const int sp = gemm::auto_splits((int)tiles, (int)(p.ldl / dx_bk(s.es)), p.ksplit);
-    t += F / Rg * q * waves(tiles * sp) * (p.wt ? 1.0 : pen);
+    t += F / Rg * q * waves(tiles * sp);
     if (sp > 1) t += nch * 2.0 * sp * (double)p.C * Hp * 4 / Rm;
-    t += F / Rg * waves(cdiv(s.V, 256) * cdiv(p.Hp, 256)) * (p.dt ? 1.0 : pen);
+    t += F / Rg * waves(cdiv(s.V, 256) * cdiv(p.Hp, 256));
     double rmw = es * V * Hp;
     if (p.dw == kDwAcc && p.nch > 1) rmw = 8.0 * V * Hp * (nch - 1) + es * V * Hp;
     if (p.dw == kDwOut) rmw = es * V * Hp * (2 * nch - 1);
     t += rmw / Rm;
     if (p.wt) t += 2.0 * es * V * Hp / Rm;
-    if (p.dt) t += 2.0 * es * BT * (double)p.V8 / Rm;
-    t += 2.0 * es * BT * Hp / Rm + nch * 4 * launch;
+    if (p.dt) t += 2.0 * es * BT * ((double)p.V8 + Hp) / Rm + nch * 2 * launch;
+    t += nch * 2 * launch;
   }
   return t;
 }
@@ -956,8 +961,10 @@ bool forced_form(int* dw, bool* wt, bool* dt, int64_t* vt, bool* bad) {
 constexpr size_t kSmallWorkspace = (size_t)40 << 20;
 
 // A plan that sums dW (and dX) in fp32 is taken over a faster one that sums in
-// the 16-bit output unless it is modelled this much slower.
-constexpr double kExactSlack = 1.5;
+// the 16-bit output unless it is modelled this much slower. Vocabulary tiles
+// wider than 8192 columns, for few rows: their GEMMs have few workgroups, and
+// beyond 1.3 a call got slower (1024 rows, H 1024, V 50257: 1.26 -> 1.41 ms).
+constexpr double kExactSlack = 1.5, kWideTileSlack = 1.3;
 
 // dW summed in fp32 (or computed whole): every form but accumulation in a
 // 16-bit output over several chunks.
@@ -980,26 +987,33 @@ int fl_plan(const FlShape& s, int64_t budget, FlPlan* out) {
   const int64_t cmax_rows = std::min<int64_t>(8192, s.chunk_cap > 0 ? s.chunk_cap : 8192);
   const int64_t cmax = std::max<int64_t>(8, std::min<int64_t>(cmax_rows & ~(int64_t)7, pad8(std::max<int64_t>(s.BT, 1))));
   const int smax_full = s.grad ? (int)std::max<int64_t>(1, std::min<int64_t>(8, pad64(s.V) / dx_bk(s.es) / 16)) : 1;
-  auto lean = [&](int64_t C, int sm) {
+  auto lean = [&](int64_t C) {
     const bool mn_ok = s.es == 2;
-    return fl_layout(s, C, !mn_ok, !mn_ok, kDwOut, sm);
+    return fl_layout(s, C, !mn_ok, !mn_ok, kDwOut, 1, 0);
   };
   size_t cap;
   if (budget == 0) {
     const int64_t C0 = std::min<int64_t>(cmax, ref_chunk(s.BT, s.H, s.V));
-    // the reference's chunk logits, the gathered rows and their transpose, and an
+    // the reference's chunk logits, the gathered rows and as much again, and an
     // eighth of the chunk's bytes for the dX GEMM's split partials
-    const FlPlan b = lean(C0, 1);
-    cap = std::max({kSmallWorkspace, s.default_floor, b.total + (size_t)C0 * pad64(s.V) * s.es / 8});
+    const FlPlan b = lean(C0);
+    const size_t rows = s.grad && !b.dt ? (size_t)b.Hp * ld_t(C0) * s.es : 0;
+    cap = std::max({kSmallWorkspace, s.default_floor, b.total + rows + (size_t)C0 * pad64(s.V) * s.es / 8});
   } else {
     cap = budget < 0 ? SIZE_MAX : (size_t)budget;
   }
+  // Without a limit a FusedLinearCE call of several chunks keeps its documented plan: W^T, every chunk's D^T and
+  // one dW GEMM, with the workspace callers size for it (C5: 39.0 ms; W, D and X read MN-contiguous with an
+  // fp32 dW accumulator 38.4 ms, W alone MN-contiguous 38.2). Small hidden sizes, whose accumulator is cheap,
+  // were and stay the model's choice (16384 rows, H 1024, V 32000: 3.53 ms materialised, 3.15 accumulated).
+  const bool materialise = budget < 0 && s.ce && s.grad && !forced && s.BT > cmax && (s.H >= 2048 || s.chunk_cap > 0);
   // the fastest candidate overall, the fastest whose dW (and dX) are summed in fp32, and (fp16 inputs) the
   // fastest that does not sum dW in the fp16 output over several chunks: gradients scaled by 1/n sit in
   // fp16's subnormal range there, where each rounding costs percent-level error (the vocabulary-tiled plan
   // sums dX unscaled, which stays in the normal range)
-  bool found = false, found_ex = false, found_safe = false;
-  FlPlan best, best_ex, best_safe;
+  bool found = false, found_safe = false;
+  bool found_ex[2] = {false, false};  // tiles of at most 8192 columns and row chunks; wider tiles
+  FlPlan best, best_ex[2], best_safe;
   auto consider = [&](const FlPlan& p) {
     auto better = [&](const FlPlan& a, const FlPlan& b) {
       return a.cost < b.cost || (a.cost == b.cost && a.total < b.total);
@@ -1008,9 +1022,10 @@ int fl_plan(const FlShape& s, int64_t budget, FlPlan* out) {
       best = p;
       found = true;
     }
-    if (exact_dw(s, p) && (!found_ex || better(p, best_ex))) {
-      best_ex = p;
-      found_ex = true;
+    const int wide = p.vtile && p.Vt > 8192;
+    if (exact_dw(s, p) && (!found_ex[wide] || better(p, best_ex[wide]))) {
+      best_ex[wide] = p;
+      found_ex[wide] = true;
     }
     const bool risky = s.f16 && !p.vtile && !exact_dw(s, p);
     if (!risky && (!found_safe || better(p, best_safe))) {
@@ -1025,10 +1040,15 @@ int fl_plan(const FlShape& s, int64_t budget, FlPlan* out) {
   }
   for (int64_t C : cs) {
     const int64_t nch = s.BT > 0 ? cdiv(s.BT, C) : 0;
+    size_t part[4] = {0, 0, 0, 0};  // the partials' bytes at each split cap below
+    if (s.grad)
+      for (int sm = smax_full, i = 0; sm >= 1; sm = sm > 1 ? sm / 2 : 0, ++i)
+        part[i] = dx_part_bytes(C, pad8(s.H), pad64(s.V), dx_bk(s.es), sm);
     fl_forms(s, nch, [&](bool wt, bool dt, int dw) {
       if (forced && (f_vt > 0 || dw != f_dw || wt != f_wt || dt != f_dt)) return;
-      for (int sm = smax_full; sm >= 1; sm = sm > 1 ? sm / 2 : 0) {
-        FlPlan p = fl_layout(s, C, wt, dt, dw, sm);
+      if (materialise && !(wt && dt && dw == kDwDefer)) return;
+      for (int sm = smax_full, i = 0; sm >= 1; sm = sm > 1 ? sm / 2 : 0, ++i) {
+        FlPlan p = fl_layout(s, C, wt, dt, dw, sm, part[i]);
         if (p.total > cap) continue;
         p.cost = fl_cost(s, p);
         consider(p);
@@ -1037,8 +1057,10 @@ int fl_plan(const FlShape& s, int64_t budget, FlPlan* out) {
     });
   }
   if (s.vt_ok && s.BT > 0 && (forced ? f_vt > 0 : s.chunk_cap <= 0)) {
-    const int64_t vmax = std::min<int64_t>(8192, (s.V + 255) / 256 * 256);
-    for (int64_t Vt = vmax; Vt >= 256; Vt -= 256)
+    // tiles of up to the whole vocabulary (above 8192 columns in steps of 2048): few rows need wide tiles to
+    // fill the chip (500 rows of V 128256: a GEMM of 8192 columns has 64 workgroups)
+    const int64_t vmax = (s.V + 255) / 256 * 256;
+    for (int64_t Vt = vmax; Vt >= 256 && !materialise; Vt = Vt > 8192 ? std::max<int64_t>(8192, (Vt - 1) / 2048 * 2048) : Vt - 256)
       for (int dw : {kDwAcc, kDwOut}) {
         if (forced && (Vt != f_vt || dw != f_dw)) continue;
         FlPlan p = vt_layout(s, Vt, dw);
@@ -1052,14 +1074,20 @@ int fl_plan(const FlShape& s, int64_t budget, FlPlan* out) {
     return HK_EINVAL;
   }
   if (!found) {
-    const FlPlan small = lean(cs.back(), 1);
+    const FlPlan small = lean(cs.back());
     set_error("workspace budget %lld bytes is below the smallest plan (%zu bytes)", (long long)budget, small.total);
     return HK_EINVAL;
   }
   // fp32 sums unless they cost more than half as much time again as the fastest plan (fp16: the fastest
   // plan without fp16 dW sums over chunks, when one fits)
   const FlPlan& fast = s.f16 && found_safe ? best_safe : best;
-  *out = found_ex && best_ex.cost <= kExactSlack * fast.cost ? best_ex : fast;
+  const FlPlan* take = nullptr;
+  for (int wide = 0; wide < 2; ++wide) {
+    const FlPlan& e = best_ex[wide];
+    if (found_ex[wide] && e.cost <= (wide ? kWideTileSlack : kExactSlack) * fast.cost && (!take || e.cost < take->cost))
+      take = &e;
+  }
+  *out = take ? *take : fast;
   return HK_OK;
 }
 
@@ -1089,7 +1117,7 @@ int chunked_lm_head(const T* X, const T* W, int64_t BT, int64_t H, int64_t V, ch
   T* Xg = p.gather ? (T*)(ws + p.xg) : nullptr;
   T* Wp = p.wpad ? (T*)(ws + p.wp) : nullptr;
   T* Wt = p.wt ? (T*)(ws + p.wtp) : nullptr;
-  T* Xt = grad ? (T*)(ws + p.xt) : nullptr;
+  T* Xt = p.dt ? (T*)(ws + p.xt) : nullptr;
   T* Dt = p.dt ? (T*)(ws + p.dtp) : nullptr;
   float* acc = (grad && p.dw == kDwAcc) ? (float*)(ws + p.acc) : nullptr;
   const T* Wk = p.wpad ? Wp : W;  // K-contiguous weight rows
@@ -1163,22 +1191,21 @@ int chunked_lm_head(const T* X, const T* W, int64_t BT, int64_t H, int64_t V, ch
     rc = row_step(Lg, r0, cs);
     if (rc) return rc;
     if (!grad) continue;
-    // X_c^T (zeros past the live rows) into X^T: columns [r0, r0 + cs) of [Hp, BT] when
-    // deferred, else [Hp, C]; and D_c^T when materialised: into columns [r0, r0 + cs) of
-    // D^T [V8, BTp] (zeros past the live rows) when deferred, else D^T [V8, C]. On the
-    // side stream, beside the dX GEMM, which also only reads the chunk.
+    // With D^T materialised: X_c^T (zeros past the live rows) into X^T, columns [r0, r0 + cs) of [Hp, BT] when
+    // deferred, else [Hp, C], and D_c^T into D^T, columns [r0, r0 + cs) of [V8, BTp] (zeros past the live
+    // rows) when deferred, else [V8, C]. On the side stream, beside the dX GEMM, which also only reads the
+    // chunk.
     const int64_t csp = pad8(cs);
-    {
-      rc = join();  // W^T, which the dX GEMM reads
-      if (rc) return rc;
+    rc = join();  // W^T, which the dX GEMM reads
+    if (rc) return rc;
+    if (p.dt) {
       rc = fork();
       if (rc) return rc;
       T* xt_dst = defer ? Xt + r0 : Xt;
       const int64_t xrp = defer ? (ci + 1 < p.nch ? cs : BTp - r0) : csp;
       rc = launch_transpose<T>(xt_dst, Xc, cs, xrp, Hp, ldxc, ldxt, side, n_live, r0);
       if (rc) return rc;
-      if (defer) rc = launch_transpose<T>(Dt + r0, Lg, cs, xrp, p.V8, ldl, ldxt, side, n_live, r0);
-      else if (p.dt) rc = launch_transpose<T>(Dt, Lg, cs, csp, p.V8, ldl, ldxt, side, n_live, r0);
+      rc = launch_transpose<T>(defer ? Dt + r0 : Dt, Lg, cs, xrp, p.V8, ldl, ldxt, side, n_live, r0);
       if (rc) return rc;
       side_pending = true;
     }
@@ -1203,17 +1230,18 @@ int chunked_lm_head(const T* X, const T* W, int64_t BT, int64_t H, int64_t V, ch
       if (rc) return rc;
     }
     if (defer) continue;
-    // dW (+)= D_c^T X_c; K = cs is padded to a multiple of 8 with zeros on both operands, and cut
-    // on the device to the live rows
+    // dW (+)= D_c^T X_c, K (= cs) cut on the device to the live rows; transposed operands are padded to a
+    // multiple of 8 with zeros
     rc = join();
     if (rc) return rc;
     auto dw_gemm = [&](auto epi) {
       if (p.dt)
         return launch_gemm<T>(Dt, Xt, (int)V, (int)Hp, (int)csp, ldxt, ldxt, epi, st, n_live, (int)r0, true);
-      // D_c [cs, ldl] read MN-contiguous (k = the chunk row, m = the vocabulary column); its rows stop at
-      // cs (the chunk buffer's rows past it were never written), or at the live rows on the device
-      return launch_gemm_mn<T, true, false>(Lg, Xt, (int)p.V8, (int)Hp, (int)csp, ldl, ldxt, epi, st, n_live,
-                                            (int)r0, true, 1, 0, (int)cs);
+      // D_c [cs, ldl] (k = the chunk row, m = the vocabulary column) and X_c [cs, Hp] (n = the hidden column)
+      // read MN-contiguous; their rows stop at cs (the chunk buffer's rows past it were never written), or at
+      // the live rows on the device
+      return launch_gemm_mn<T, true, true>(Lg, Xc, (int)p.V8, (int)Hp, (int)cs, ldl, ldxc, epi, st, n_live, (int)r0,
+                                           true, 1, (int)cs, (int)cs);
     };
     const int vl = (int)V, hl = (int)H;
     if (p.nch == 1) rc = dw_gemm(EpiDw<T, 0>{dWo, H, nullptr, Hp, vl, hl, wvec});
