@@ -82,6 +82,36 @@ __device__ __forceinline__ f32x4_t load4(const T* p, int n, bool vec) {
   return x;
 }
 
+// 8-column forms of the two (gemm_wide.h's epilogue): vec 2 (the address is 16-byte aligned in 16-bit T) moves 16
+// bytes at a time, vec 1 (8-byte aligned) 8. The loaded values stay packed.
+template <typename T>
+__device__ __forceinline__ void store8(T* p, const float* v, int n, int vec) {
+  if constexpr (sizeof(T) == 2) {
+    if (n == 8 && vec == 2) {
+      *reinterpret_cast<u32x4*>(p) = u32x4{gemm::pack2<T>(v[0], v[1]), gemm::pack2<T>(v[2], v[3]),
+                                           gemm::pack2<T>(v[4], v[5]), gemm::pack2<T>(v[6], v[7])};
+      return;
+    }
+  }
+  store4<T>(p, v, min(n, 4), vec != 0);
+  if (n > 4) store4<T>(p + 4, v + 4, n - 4, vec != 0);
+}
+template <typename T>
+struct alignas(16) Row8 {
+  T v[8];
+};
+template <typename T>
+__device__ __forceinline__ Row8<T> load8(const T* p, int n, int vec) {
+  Row8<T> x;
+  if (n == 8 && vec == 2) {
+    x = *reinterpret_cast<const Row8<T>*>(p);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x.v[e] = e < n ? p[e] : from_f32<T>(0.f);
+  }
+  return x;
+}
+
 // The logits GEMM's epilogue: C (T) = acc in 16-byte chunks (ldc a multiple of
 // 8, C 16-byte aligned). The chunk that straddles column N is completed with
 // `pad` past N: -inf for the CrossEntropy and GRPO row steps, which then read
@@ -106,6 +136,18 @@ struct EpiLogits {
       for (int e = 0; e < E; ++e) p[e] = e < n ? v[e] : fill;
     }
   }
+  using Prior8 = NoPrior;
+  __device__ __forceinline__ int64_t out_row(int row) const { return row; }
+  __device__ __forceinline__ void store8(int64_t out, int col, const float* v, int n, const Prior8&) const {
+    T* p = C + out * ldc + col;
+    if (n == 8) {
+      hk::store8<T>(p, v, 8, 2);
+    } else {
+      const T fill = from_f32<T>(pad);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) p[e] = e < n ? from_f32<T>(v[e]) : fill;
+    }
+  }
 };
 
 // The dX GEMM's epilogue (M = chunk rows, N = the padded hidden size). GEMM row
@@ -124,7 +166,7 @@ struct EpiDx {
   float* part;
   int64_t ld;   // a multiple of 4
   int cols;
-  bool vec;     // C rows 8-byte (16-bit) / 16-byte (fp32) aligned at every 4th column
+  int vec;      // C rows 8-byte (16-bit) / 16-byte (fp32) aligned at every 4th column (1), and 16-byte at every 8th (2)
   int split = 0, nsplit = 1, m = 0;
   __device__ __forceinline__ void set_split(int s, int ns, int bounded_m) {
     split = s;
@@ -135,14 +177,21 @@ struct EpiDx {
   __device__ __forceinline__ void store(int row, int col, const float* v, int n, const Prior&) const {
     if (nsplit == 1) {
       n = min(n, cols - col);
-      if (n > 0) store4<T>(C + (int64_t)(rows ? rows[row] : row) * ldc + col, v, n, vec);
+      if (n > 0) store4<T>(C + (int64_t)(rows ? rows[row] : row) * ldc + col, v, n, vec != 0);
       return;
     }
-    float* p = part + ((int64_t)split * m + row) * ld + col;
-    if (n == 4) {
-      *reinterpret_cast<f32x4_t*>(p) = f32x4_t{v[0], v[1], v[2], v[3]};
+    store4<float>(part + ((int64_t)split * m + row) * ld + col, v, n, true);
+  }
+  using Prior8 = NoPrior;
+  __device__ __forceinline__ int64_t out_row(int row) const {
+    return nsplit > 1 ? (int64_t)split * m + row : rows ? rows[row] : row;
+  }
+  __device__ __forceinline__ void store8(int64_t out, int col, const float* v, int n, const Prior8&) const {
+    if (nsplit == 1) {
+      n = min(n, cols - col);
+      if (n > 0) hk::store8<T>(C + out * ldc + col, v, n, vec);
     } else {
-      for (int e = 0; e < n; ++e) p[e] = v[e];
+      hk::store8<float>(part + out * ld + col, v, n, 1);
     }
   }
 };
@@ -163,12 +212,12 @@ struct EpiDw {
   float* acc;
   int64_t lda;  // a multiple of 4
   int rows_lim, cols_lim;
-  bool vec;     // out rows aligned for 4-element stores
+  int vec;      // out rows aligned for 4-element stores (1), for 16-byte ones in 16-bit T (2)
   const int* inv_n = nullptr;  // nullable: the values are multiplied by 1 / max(*inv_n, 1) first
   __device__ __forceinline__ Prior load(int row, int col, int n) const {
     if (row >= rows_lim || col >= cols_lim) return Prior{0.f, 0.f, 0.f, 0.f};
     n = min(n, cols_lim - col);
-    if constexpr (MODE == 1) return load4<T>(out + (int64_t)row * ldo + col, n, vec);
+    if constexpr (MODE == 1) return load4<T>(out + (int64_t)row * ldo + col, n, vec != 0);
     const float* p = acc + (int64_t)row * lda + col;
     if (n == 4) return *reinterpret_cast<const f32x4_t*>(p);
     Prior x = {0.f, 0.f, 0.f, 0.f};
@@ -190,8 +239,30 @@ struct EpiDw {
         for (int e = 0; e < n; ++e) p[e] = r[e];
       }
     } else {
-      store4<T>(out + (int64_t)row * ldo + col, r, n, vec);
+      store4<T>(out + (int64_t)row * ldo + col, r, n, vec != 0);
     }
+  }
+  using Prior8 = Row8<typename std::conditional<MODE == 1, T, float>::type>;
+  __device__ __forceinline__ int64_t out_row(int row) const { return row; }
+  __device__ __forceinline__ Prior8 load8(int64_t row, int col, int n) const {
+    n = row < rows_lim ? min(n, cols_lim - col) : 0;
+    if constexpr (MODE == 1) return hk::load8<T>(out + row * ldo + col, n, vec);
+    else return hk::load8<float>(acc + row * lda + col, n, 2);
+  }
+  __device__ __forceinline__ void store8(int64_t row, int col, const float* v, int n, const Prior8& x) const {
+    if (row >= rows_lim || col >= cols_lim) return;
+    n = min(n, cols_lim - col);
+    const float f = inv_n ? 1.f / (float)max(*inv_n, 1) : 1.f;
+    float r[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float prior = 0.f;
+      if constexpr (MODE == 1) prior = to_f32<T>(x.v[e]);
+      else if constexpr (kReads) prior = x.v[e];
+      r[e] = prior + v[e] * f;
+    }
+    if constexpr (MODE == 2 || MODE == 3) hk::store8<float>(acc + row * lda + col, r, n, 1);
+    else hk::store8<T>(out + row * ldo + col, r, n, vec);
   }
 };
 
@@ -1165,8 +1236,9 @@ int chunked_lm_head(const T* X, const T* W, int64_t BT, int64_t H, int64_t V, ch
     side_pending = true;
   }
   const int64_t BTp = pad8(BT), ldxt = ld_t(defer ? BT : C);
-  const bool dvec = H % 4 == 0 && aligned_to(dX, 16);    // 4-element stores of dX rows
-  const bool wvec = H % 4 == 0 && aligned_to(dWo, 16);   // and of dW rows
+  // 4- and 8-element stores of dX and of dW rows
+  const int dvec = !aligned_to(dX, 16) ? 0 : H % 8 == 0 ? 2 : H % 4 == 0 ? 1 : 0;
+  const int wvec = !aligned_to(dWo, 16) ? 0 : H % 8 == 0 ? 2 : H % 4 == 0 ? 1 : 0;
   const int kt_dx = (int)(ldl / gemm::CfgFor<T>::BK);
   for (int64_t ci = 0; ci < p.nch; ++ci) {
     const int64_t r0 = ci * C;
@@ -1323,8 +1395,8 @@ int vtiled_ce(const T* X, const T* W, int64_t BT, int64_t H, int64_t V, char* ws
                      state, loss_rows, targets, ignore_index, n_valid, scale ? 1 : 0, BT);
   rc = check_launch("vt_finalize_kernel");
   if (rc || !grad) return rc;
-  const bool dvec = H % 4 == 0 && aligned_to(dX, 16);
-  const bool wvec = H % 4 == 0 && aligned_to(dWo, 16);
+  const int dvec = !aligned_to(dX, 16) ? 0 : H % 8 == 0 ? 2 : H % 4 == 0 ? 1 : 0;
+  const int wvec = !aligned_to(dWo, 16) ? 0 : H % 8 == 0 ? 2 : H % 4 == 0 ? 1 : 0;
   // dX summed in the output over several tiles: D without the 1/n of 'mean' (applied by dW's epilogue and
   // by the last pass over dX), and without its target entries (see vt_drop_targets_kernel)
   const bool out_sum = p.ntiles > 1 && !acc;

@@ -839,8 +839,11 @@ int launch(const T* A, const T* B, int M, int N, int K, int64_t lda, int64_t ldb
   if (a_ok && b_ok) {
     if constexpr (sizeof(T) == 2) {
       static_assert(C::BM == Wide::BM && C::BN == Wide::BN && C::BK == Wide::BK, "one tile for both kernels' grids");
-      hipLaunchKernelGGL((gemm_wide_kernel<T, Epi, AMN, BMN>), dim3((unsigned)blocks), dim3(Wide::NT), 0, st, A, B, g,
-                         epi);
+      // persistent: one workgroup a CU (its LDS and registers allow no second one), a multiple of the 8 XCDs
+      const int dev = current_device();
+      const int cus = dev >= 0 ? cu_count(dev) & ~7 : 0;
+      const unsigned grid = (unsigned)(cus > 0 && blocks > cus ? cus : blocks);
+      hipLaunchKernelGGL((gemm_wide_kernel<T, Epi, AMN, BMN>), dim3(grid), dim3(Wide::NT), 0, st, A, B, g, epi);
       return check_launch("gemm_wide_kernel");
     } else {
       hipLaunchKernelGGL((gemm_kk_kernel<T, C, Epi>), dim3((unsigned)blocks), dim3(C::NT), 0, st, A, B, g, epi);

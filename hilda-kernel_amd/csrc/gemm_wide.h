@@ -27,12 +27,17 @@
 // stages apart: hence core() and its restrict pointers, one per operand and
 // stage. (Without them every stage waited for the next one's loads.)
 //
-// Measured, TFLOP/s, kernel alone, before (8 waves) -> after; M x N x K:
-//   both K-contiguous   8192x32000x4096 1280 -> 1426   8192x4096x32000 1285 -> 1422
-//   B MN-contiguous     8192x32000x4096 1115 -> 1419   8192x4096x32000 1107 -> 1443
-//   both MN-contiguous  8192x32000x4096 1057 -> 1431   8192x4096x32000 1075 -> 1474
-// torch.matmul on the first shape, its own layout: 1494. The matrix pipes are
-// 73% busy at 1.9 GHz in all three.
+// Persistent: a workgroup walks its tiles (blockIdx.x, + gridDim.x, ..) and fetches the next tile's first two stages
+// during this one's last two, so the accumulators go out (WideOut below) while those land and no tile starts on an
+// empty pipeline.
+//
+// Measured, TFLOP/s, kernel alone, 8 waves and one tile a workgroup -> this; M x N x K:
+//   both K-contiguous                  8192x32768x4096 1280 -> 1454-1484
+//   both MN-contiguous                 8192x32768x4096 1060 -> 1373-1382   8192x4096x4096 1170 -> 1493-1524
+//   B MN-contiguous, read-modify-write 8192x4096x4096  1070 -> 1393-1458
+// A tile's time beyond its K loop (the intercept over K at 8192x32768): 13 us one tile a workgroup -> 7 us, with a
+// read-modify-write epilogue 51 -> 21 us. torch.matmul's best layout at 8192x32000x4096: 1494. In long runs the
+// matrix pipes are 73% busy at 1.9 GHz: the power limit.
 #pragma once
 
 #include "hk_common.h"
@@ -41,6 +46,10 @@
 
 namespace hk {
 namespace gemm {
+
+// A lambda inlined with the function it stands in (before that function is inlined elsewhere, where its alias
+// scopes are attached).
+#define HK_INLINE __attribute__((always_inline))
 
 struct Wide {
   static constexpr int BM = 256, BN = 256, BK = 64, NT = 256;
@@ -59,26 +68,36 @@ struct Wide {
 __device__ __forceinline__ int wide_swz_k(int row) { return (row >> 1) & 7; }
 __device__ __forceinline__ int wide_swz_mn(int k) { return (4 * (k & 3)) ^ (2 * ((k >> 3) & 1)); }
 
-// The K loop: acc += the tile's products over KT stages of 64 k.
-// a0 a1 b0 b1: the LDS stages. pa, pb: the operand panels at this workgroup's
-// first row (column) and first k. ra, rb: their rows inside the matrix. ka, kb:
-// stored k past that start (MN-contiguous operands).
-template <typename T, bool AMN, bool BMN>
-__device__ __forceinline__ void wide_core(f32x4_t (&acc)[8][8], unsigned char* __restrict__ a0,
-                                          unsigned char* __restrict__ a1, unsigned char* __restrict__ b0,
-                                          unsigned char* __restrict__ b1, const T* __restrict__ pa,
-                                          const T* __restrict__ pb, int64_t lda, int64_t ldb, int rows_a, int rows_b,
-                                          int KT, int ka, int kb, int wave, int lane) {
+// A tile's operand panels: the element offset of their first row (column) and first k, their rows inside the matrix,
+// the stored k past that start (MN-contiguous operands), and the tile's stages.
+struct WideTile {
+  int64_t at_a, at_b;
+  int rows_a, rows_b, KT, ka, kb;
+};
+
+// Every tile of this workgroup: next(tile) gives the first and each following one (false: none left), done(acc) takes
+// a finished one's accumulators, early() runs a stage before that. a0 a1 b0 b1: the LDS stages.
+template <typename T, bool AMN, bool BMN, class Next, class Early, class Done>
+__device__ __forceinline__ void wide_core(unsigned char* __restrict__ a0, unsigned char* __restrict__ a1,
+                                          unsigned char* __restrict__ b0, unsigned char* __restrict__ b1,
+                                          const T* __restrict__ A, const T* __restrict__ B, int64_t lda, int64_t ldb,
+                                          int wave, int lane, Next&& next, Early&& early, Done&& done) {
 #if defined(__HIP_DEVICE_COMPILE__)
   static_assert(sizeof(T) == 2, "bf16 or fp16 inputs");
   const int wm = wave >> 1, wn = wave & 1, fr = lane & 15, fk = lane >> 4;
-  KT = __builtin_amdgcn_readfirstlane(KT);
+  f32x4_t acc[8][8];
+  auto clear = [&]() HK_INLINE {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  };
 
   // LDS read bases. K-contiguous fragment t of half h: lane l holds row 16 t + l % 16, k = 32 h + 8 (l / 16)
   // .. + 7, one ds_read_b128 (one base per half, t in the immediate). MN-contiguous: two transposed reads (k
   // + 0..3, + 4..7); within each 16-lane group, lane i points at k-row i / 4 and row 4 (i % 4) and receives
   // row i's four k (one base per fragment, the half in the immediate).
-  auto read_base = [&](bool mn, int R, int t) -> uint32_t {
+  auto read_base = [&](bool mn, int R, int t) HK_INLINE -> uint32_t {
     if (mn) {
       const int kq = fr >> 2, r = R + 16 * t + 4 * (fr & 3), k = 8 * fk + kq;
       return (uint32_t)((k * 256 + ((r >> 3) ^ wide_swz_mn(k)) * 8 + (r & 7)) * 2);
@@ -102,7 +121,7 @@ __device__ __forceinline__ void wide_core(f32x4_t (&acc)[8][8], unsigned char* _
   // the buffer's end. MN-contiguous: the buffer starts at the stage's first k-row and ends with the stored
   // k-rows; chunks past the matrix's rows are redirected out of it.
   uint32_t va[8], vb[8];
-  auto dma_offset = [&](bool mn, int q, int64_t ld, int rows) -> uint32_t {
+  auto dma_offset = [&](bool mn, int q, int64_t ld, int rows) HK_INLINE -> uint32_t {
     if (mn) {
       const int k = q / 32, r = ((q % 32) ^ wide_swz_mn(k)) * 8;
       return r < rows ? (uint32_t)(k * ld + r) * 2u : kOobOffset;
@@ -110,44 +129,49 @@ __device__ __forceinline__ void wide_core(f32x4_t (&acc)[8][8], unsigned char* _
     const int r = q / 8;
     return (uint32_t)(r * ld + ((q % 8) ^ wide_swz_k(r)) * 8) * 2u;
   };
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    va[i] = dma_offset(AMN, (wave * 8 + i) * 64 + lane, lda, rows_a);
-    vb[i] = dma_offset(BMN, (wave * 8 + i) * 64 + lane, ldb, rows_b);
-  }
   // one operand's next stage: its buffer and scalar offset, advanced a stage per call. Scalar values only
   // (readfirstlane): a buffer in vector registers would turn every load into a loop over its lanes.
-  struct Next {
-    const char* p;
-    int64_t step;
-    int ld2, left, off;
+  // (the pointer is the kernel's argument plus a scalar offset: its alias scope has to be seen, too.)
+  struct Feed {
+    int64_t at;  // bytes
+    int left, off, bytes;
   };
-  auto scalar = [](const char* p) {
-    const uint64_t v = (uint64_t)p;
-    return const_cast<char*>(reinterpret_cast<const char*>(
-        (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v) |
-        ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32)));
+  auto scalar = [](int64_t v) HK_INLINE {
+    return (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v) |
+                     ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)((uint64_t)v >> 32)) << 32));
   };
-  const int bytes_a = AMN ? 0 : (int)(rows_a * lda * 2), bytes_b = BMN ? 0 : (int)(rows_b * ldb * 2);
-  // (an MN-contiguous operand of an odd stage count ends at KT stages: the trailing one reads zeros)
-  Next na{(const char*)pa, 64 * lda * 2, (int)lda * 2, __builtin_amdgcn_readfirstlane(AMN ? min(ka, KT * 64) : KT * 64),
-          -128};
-  Next nb{(const char*)pb, 64 * ldb * 2, (int)ldb * 2, __builtin_amdgcn_readfirstlane(BMN ? min(kb, KT * 64) : KT * 64),
-          -128};
+  Feed na{}, nb{};
+  // the feeds at a tile's start; without one (`any` false) they end at once and their loads return zeros
+  auto feed = [&](const WideTile& t, bool any) HK_INLINE {
+    // (an MN-contiguous operand of an odd stage count ends at KT stages: the trailing one reads zeros)
+    na = Feed{scalar(t.at_a * 2),
+              __builtin_amdgcn_readfirstlane(any ? (AMN ? min(t.ka, t.KT * 64) : t.KT * 64) : 0), -128,
+              AMN ? (int)lda * 2 : __builtin_amdgcn_readfirstlane((int)(t.rows_a * lda * 2))};
+    nb = Feed{scalar(t.at_b * 2),
+              __builtin_amdgcn_readfirstlane(any ? (BMN ? min(t.kb, t.KT * 64) : t.KT * 64) : 0), -128,
+              BMN ? (int)ldb * 2 : __builtin_amdgcn_readfirstlane((int)(t.rows_b * ldb * 2))};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      va[i] = dma_offset(AMN, (wave * 8 + i) * 64 + lane, lda, t.rows_a);
+      vb[i] = dma_offset(BMN, (wave * 8 + i) * 64 + lane, ldb, t.rows_b);
+    }
+  };
   __amdgpu_buffer_rsrc_t rsa, rsb;
-  auto setup = [&](bool mn, Next& n, int panel_bytes, __amdgpu_buffer_rsrc_t& rs) {
-    if (mn) {
-      const int bytes = __builtin_amdgcn_readfirstlane(max(0, min(64, n.left)) * n.ld2);
-      rs = __builtin_amdgcn_make_buffer_rsrc(scalar(n.p), 0, bytes, kRsrcWord3);
-      n.p += n.step;
+  auto setup = [&](bool mn, Feed& n, const T* p, int64_t ld, __amdgpu_buffer_rsrc_t& rs) HK_INLINE {
+    char* const base = const_cast<char*>(reinterpret_cast<const char*>(p)) + scalar(n.at);
+    if (mn) {  // n.bytes: a k-row's
+      const int bytes = __builtin_amdgcn_readfirstlane(max(0, min(64, n.left)) * n.bytes);
+      rs = __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, kRsrcWord3);
+      n.at += 128 * ld;
       n.off = 0;
-    } else {  // past the last stage: a zero-length buffer, the loads return zeros
-      rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(n.p), 0, n.left > 0 ? panel_bytes : 0, kRsrcWord3);
+    } else {  // n.bytes: the panel's; past the last stage a zero-length buffer, the loads return zeros
+      rs = __builtin_amdgcn_make_buffer_rsrc(base, 0, __builtin_amdgcn_readfirstlane(n.left > 0 ? n.bytes : 0),
+                                             kRsrcWord3);
       n.off = n.left > 0 ? n.off + 128 : 0;
     }
     n.left -= 64;
   };
-  auto dma = [&](auto stage, int t) {  // load t (A 0..7, B 8..15) of the stage set up last
+  auto dma = [&](auto stage, int t) HK_INLINE {  // load t (A 0..7, B 8..15) of the stage set up last
     constexpr int st = decltype(stage)::value;
     if (t < 8)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (st ? a1 : a0) + (wave * 8 + t) * 1024, 16, va[t], na.off, 0, 0);
@@ -158,7 +182,7 @@ __device__ __forceinline__ void wide_core(f32x4_t (&acc)[8][8], unsigned char* _
 
   typedef short v4i16 __attribute__((ext_vector_type(4)));
   typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
-  auto frag = [&](bool mn, unsigned char* p, uint32_t base_t, uint32_t base_h, int h, int t) -> u32x4 {
+  auto frag = [&](bool mn, unsigned char* p, uint32_t base_t, uint32_t base_h, int h, int t) HK_INLINE -> u32x4 {
     if (mn) {
       v4i16 v[2];
 #pragma unroll
@@ -171,7 +195,7 @@ __device__ __forceinline__ void wide_core(f32x4_t (&acc)[8][8], unsigned char* _
   };
   u32x4 fa[2][8], fb[2][8];
   // read s (0..15) of half h, in the order the MFMAs need them: b0 a0 b1 .. b7 a1 .. a7
-  auto read = [&](auto stage, int h, int s) {
+  auto read = [&](auto stage, int h, int s) HK_INLINE {
     constexpr int st = decltype(stage)::value;
     const bool is_b = s == 0 || (s >= 2 && s <= 8);
     const int t = s <= 1 ? 0 : s <= 8 ? s - 1 : s - 8;
@@ -179,7 +203,7 @@ __device__ __forceinline__ void wide_core(f32x4_t (&acc)[8][8], unsigned char* _
     else fa[h][t] = frag(AMN, st ? a1 : a0, abase[AMN ? t : 0], abase[AMN ? 0 : h], h, t);
   };
   // MFMA m of half h: fed B then A, so a lane holds C row 16 i + l % 16, columns 16 j + 4 (l / 16) .. + 3
-  auto mma = [&](int h, int m) {
+  auto mma = [&](int h, int m) HK_INLINE {
     const int i = m >> 3, j = m & 7;
     if constexpr (std::is_same<T, __bf16>::value)
       asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(fb[h][j]), "v"(fa[h][i]));
@@ -188,7 +212,7 @@ __device__ __forceinline__ void wide_core(f32x4_t (&acc)[8][8], unsigned char* _
   };
   // The compiler does not know the asm above as MFMAs: before their first use and after their last, every
   // accumulator waits out the longest MFMA hazard.
-  auto settle = [&]() {
+  auto settle = [&]() HK_INLINE {
 #pragma unroll
     for (int i = 0; i < 8; ++i)
       asm volatile("s_nop 15"
@@ -196,7 +220,7 @@ __device__ __forceinline__ void wide_core(f32x4_t (&acc)[8][8], unsigned char* _
                      "+a"(acc[i][5]), "+a"(acc[i][6]), "+a"(acc[i][7]));
   };
   // s_waitcnt as an instruction the compiler counts (asm text it would not)
-  auto wait = [](auto cnt) {
+  auto wait = [](auto cnt) HK_INLINE {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(decltype(cnt)::value);
     asm volatile("" ::: "memory");
@@ -204,7 +228,7 @@ __device__ __forceinline__ void wide_core(f32x4_t (&acc)[8][8], unsigned char* _
   using Lgkm0 = std::integral_constant<int, 0xc07f>;
   using Vm0Lgkm0 = std::integral_constant<int, 0x0070>;
   using Vm16 = std::integral_constant<int, 0x4f70>;
-  auto barrier = []() {
+  auto barrier = []() HK_INLINE {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -212,15 +236,15 @@ __device__ __forceinline__ void wide_core(f32x4_t (&acc)[8][8], unsigned char* _
   using S0 = std::integral_constant<int, 0>;
   using S1 = std::integral_constant<int, 1>;
 
-  auto body = [&](auto cur) {
+  auto body = [&](auto cur) HK_INLINE {
     using Nx = std::integral_constant<int, decltype(cur)::value ^ 1>;
     wait(Lgkm0{});
 #pragma unroll
     for (int m = 0; m < 64; ++m) {
       mma(0, m);
       if (m % Wide::kRead1 == 0 && m / Wide::kRead1 < 16) read(cur, 1, m / Wide::kRead1);
-      if (m == Wide::kSetupA) setup(AMN, na, bytes_a, rsa);
-      if (m == Wide::kSetupB) setup(BMN, nb, bytes_b, rsb);
+      if (m == Wide::kSetupA) setup(AMN, na, A, lda, rsa);
+      if (m == Wide::kSetupB) setup(BMN, nb, B, ldb, rsb);
     }
     wait(Vm0Lgkm0{});  // this wave's DMA of the next stage, and its reads of this one
     barrier();         // every wave's
@@ -232,102 +256,95 @@ __device__ __forceinline__ void wide_core(f32x4_t (&acc)[8][8], unsigned char* _
     }
   };
 
-  settle();
-  setup(AMN, na, bytes_a, rsa);
-  setup(BMN, nb, bytes_b, rsb);
+  WideTile cur;
+  if (!next(cur)) return;
+  feed(cur, true);
+  setup(AMN, na, A, lda, rsa);
+  setup(BMN, nb, B, ldb, rsb);
 #pragma unroll
   for (int t = 0; t < 16; ++t) dma(S0{}, t);
-  setup(AMN, na, bytes_a, rsa);
-  setup(BMN, nb, bytes_b, rsb);
+  setup(AMN, na, A, lda, rsa);
+  setup(BMN, nb, B, ldb, rsb);
 #pragma unroll
   for (int t = 0; t < 16; ++t) dma(S1{}, t);
   wait(Vm16{});  // stage 0
   barrier();
 #pragma unroll
   for (int s = 0; s < 16; ++s) read(S0{}, 0, s);
-  const int KT2 = KT + (KT & 1);  // an odd count gets a trailing stage of zeros
-  for (int kt = 0; kt + 2 < KT2; kt += 2) {
+  for (bool more = true; more;) {
+    clear();
+    settle();
+    // an odd stage count gets a trailing stage of zeros
+    for (int kt = (__builtin_amdgcn_readfirstlane(cur.KT) + 1) / 2; kt > 1; --kt) {
+      body(S0{});
+      body(S1{});
+    }
+    // the tile's last two stages, fetching the next tile's first two; the accumulators go out while those land
+    more = next(cur);
+    feed(cur, more);
+    early();
     body(S0{});
     body(S1{});
+    settle();
+    done(acc);
   }
-  body(S0{});
-  wait(Lgkm0{});
-#pragma unroll
-  for (int m = 0; m < 64; ++m) {
-    mma(0, m);
-    if (m < 16) read(S1{}, 1, m);
-  }
-#pragma unroll
-  for (int m = 0; m < 64; ++m) mma(1, m);
-  settle();
-  wait(Vm0Lgkm0{});  // the zero-length loads past the end target LDS too: drained before it is reused
-  barrier();
+  wait(Vm0Lgkm0{});  // the zero-length loads past the end target LDS: landed before the workgroup ends
 #endif
 }
 
-// The epilogue contract of gemm_nt.h, from this kernel's accumulators: half a
-// tile (the 128 rows of two waves) is staged in LDS at a time, its 16-byte
-// chunks XOR-swizzled by the row, and read back as row chunks.
+// A finished 128x128 wave tile goes out from the accumulators, with no LDS (the next tile's stages land there) and no
+// barrier: a lane holds 4 consecutive columns of a row, two half- and quarter-wave swaps make that 8. An epilogue
+// functor takes them in
+//   static constexpr bool kReads; using Prior8 = what load8 returns;
+//   int64_t out_row(int row) const;                                              // where a row goes
+//   Prior8 load8(int64_t out, int col, int n) const;                             // (kReads)
+//   void store8(int64_t out, int col, const float* v, int n, const Prior8&) const;
+// with n of the 8 columns from col inside the matrix. An epilogue that reads gets the loads of kBatch chunks in
+// flight, the first batch issued a stage before the tile ends. (Staged through LDS, half a tile at a time, the
+// read-modify-write of a tile took 51 us: four round trips of 8-byte loads with the matrix pipes idle.) One code
+// path for whole and edge tiles: with two, the compiler read all 256 accumulators before their branch and spilled.
 template <class Epi>
-__device__ __forceinline__ void wide_epilogue(const f32x4_t (&acc)[8][8], unsigned char* lds_raw, int m0, int n0,
-                                              const Shape& g, const Epi& epi) {
-  using S = typename Epi::Stage;
-  constexpr int EPC = 16 / (int)sizeof(S);           // elements per chunk
-  constexpr int CPR = 256 / EPC;                     // chunks per staged row
-  constexpr int SH = sizeof(S) == 4 ? 2 : 1;         // the swizzle spreads 16 rows of 4 (2) chunks over the banks
-  constexpr int PER_T = 128 * CPR / Wide::NT, BATCH = 16;
-  static_assert(128 * 256 * sizeof(S) <= Wide::kLdsBytes && PER_T % BATCH == 0, "epilogue split");
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1, fr = lane & 15, fk = lane >> 4;
-  auto barrier = []() {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-  };
-  S* const st = reinterpret_cast<S*>(lds_raw);
-  auto at = [&](int row, int chunk) { return st + row * 256 + (chunk ^ ((row & 15) << SH)) * EPC; };
-#pragma unroll 1
-  for (int p = 0; p < 2; ++p) {
-    if (wm == p) {
+struct WideOut {
+  static constexpr int kBatch = Epi::kReads ? 32 / (int)(sizeof(typename Epi::Prior8) / 4) : 1;  // 32 registers
+  Epi e;
+  int m = 0, n = 0, row0 = 0, col0 = 0;  // the matrix; this lane's first row and column
+  typename Epi::Prior8 prior[kBatch];
+
+  __device__ __forceinline__ void load(int b) {
+    if constexpr (Epi::kReads) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int c = wn * 128 + j * 16 + fk * 4;
-          S* const d = at(i * 16 + fr, c / EPC) + c % EPC;
-          if constexpr (sizeof(S) == 4) {
-            *reinterpret_cast<f32x4_t*>(d) = acc[i][j];
-          } else {
-            *reinterpret_cast<u32x2*>(d) =
-                u32x2{pack2<S>(acc[i][j][0], acc[i][j][1]), pack2<S>(acc[i][j][2], acc[i][j][3])};
-          }
-        }
-    }
-    barrier();
-    const int rbase = m0 + p * 128;
-#pragma unroll
-    for (int b0 = 0; b0 < PER_T; b0 += BATCH) {
-      typename Epi::Prior prior[BATCH];
-      if constexpr (Epi::kReads) {
-#pragma unroll
-        for (int u = 0; u < BATCH; ++u) {
-          const int c = (b0 + u) * Wide::NT + tid, r = c / CPR, col = n0 + (c % CPR) * EPC;
-          if (rbase + r < g.M && col < g.N) prior[u] = epi.load(rbase + r, col, min(EPC, g.N - col));
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < BATCH; ++u) {
-        const int c = (b0 + u) * Wide::NT + tid, r = c / CPR, cc = c % CPR, col = n0 + cc * EPC;
-        if (rbase + r < g.M && col < g.N) {
-          const u32x4 v = *reinterpret_cast<const u32x4*>(at(r, cc));
-          epi.store(rbase + r, col, reinterpret_cast<const S*>(&v), min(EPC, g.N - col), prior[u]);
-        }
+      for (int u = 0; u < kBatch; ++u) {
+        const int c = b * kBatch + u, row = row0 + 16 * (c / 4), col = col0 + 32 * (c % 4);
+        if (row < m && col < n) prior[u] = e.load8(e.out_row(row), col, min(8, n - col));
       }
     }
-    if (p == 0) barrier();
   }
-}
+  __device__ __forceinline__ void store(const f32x4_t (&acc)[8][8]) {
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int row = row0 + 16 * i;
+      const int64_t out = row < m ? e.out_row(row) : 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int c = 4 * i + j, col = col0 + 32 * j;
+        float v[8];
+        // (whole vectors are cast: __builtin_bit_cast of one vector element reads element 0 with this compiler)
+        const u32x4 lo = __builtin_bit_cast(u32x4, acc[i][2 * j]), hi = __builtin_bit_cast(u32x4, acc[i][2 * j + 1]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const auto x = __builtin_amdgcn_permlane32_swap(lo[q], hi[q], false, false);
+          const auto y = __builtin_amdgcn_permlane16_swap(x[0], x[1], false, false);
+          v[q] = __builtin_bit_cast(float, (uint32_t)y[0]);
+          v[4 + q] = __builtin_bit_cast(float, (uint32_t)y[1]);
+        }
+        if (row < m && col < n) e.store8(out, col, v, min(8, n - col), prior[c % kBatch]);
+        if (Epi::kReads && c % kBatch == kBatch - 1 && c < 31) load(c / kBatch + 1);
+      }
+    }
+#endif
+  }
+};
 
 template <typename T, class Epi, bool AMN, bool BMN>
 __global__ __launch_bounds__(Wide::NT, 1) void gemm_wide_kernel(const T* __restrict__ A, const T* __restrict__ B,
@@ -337,35 +354,43 @@ __global__ __launch_bounds__(Wide::NT, 1) void gemm_wide_kernel(const T* __restr
   const int nbm = (g.M + Wide::BM - 1) / Wide::BM, nbn = (g.N + Wide::BN - 1) / Wide::BN;
   const int tiles = nbm * nbn;
   const int KTall = (g.K + Wide::BK - 1) / Wide::BK;  // >= 1 (checked by the launcher)
-  const int nsplit = auto_splits(tiles, KTall, g.ksplit);
-  if ((int)blockIdx.x >= tiles * nsplit) return;  // uniform: past a device-side bound
-  const int split = (int)blockIdx.x / tiles;
-  int tm, tn;
-  tile_of_block<Wide::GROUP_M>((int)blockIdx.x - split * tiles, nbm, nbn, &tm, &tn);
-  const int m0 = tm * Wide::BM, n0 = tn * Wide::BN;
-  int KT = KTall, kt0 = 0;
-  if (nsplit > 1) {  // this split's stages (auto_splits keeps every split non-empty)
-    const int per = (KTall + nsplit - 1) / nsplit;
-    kt0 = split * per;
-    KT = min(per, KTall - kt0);
-  }
-  const int64_t k0 = (int64_t)kt0 * Wide::BK;
-  const T* const pa = AMN ? A + k0 * g.lda + m0 : A + m0 * g.lda + k0;
-  const T* const pb = BMN ? B + k0 * g.ldb + n0 : B + n0 * g.ldb + k0;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-
-  f32x4_t acc[8][8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int nsplit = auto_splits(tiles, KTall, g.ksplit), total = tiles * nsplit;
+  const int per = (KTall + nsplit - 1) / nsplit;  // stages a split (auto_splits keeps every split non-empty)
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // this workgroup's tiles: blockIdx.x, + gridDim.x, ... (a multiple of 8 workgroups keeps each XCD's band)
+  int unit = (int)blockIdx.x;
+  WideOut<Epi> out{epi}, pend{epi};  // the tile in flight, the one being fetched
+  auto next = [&](WideTile& t) -> bool {
+    if (unit >= total) return false;  // uniform: past the last tile, or a device-side bound
+    const int split = unit / tiles;
+    int tm, tn;
+    tile_of_block<Wide::GROUP_M>(unit - split * tiles, nbm, nbn, &tm, &tn);
+    unit += (int)gridDim.x;
+    const int m0 = tm * Wide::BM, n0 = tn * Wide::BN, kt0 = split * per;
+    const int64_t k0 = (int64_t)kt0 * Wide::BK;
+    t.at_a = AMN ? k0 * g.lda + m0 : m0 * g.lda + k0;
+    t.at_b = BMN ? k0 * g.ldb + n0 : n0 * g.ldb + k0;
+    t.rows_a = min(Wide::BM, g.M - m0);
+    t.rows_b = min(Wide::BN, g.N - n0);
+    t.KT = min(per, KTall - kt0);
+    t.ka = g.ka - (int)k0;
+    t.kb = g.kb - (int)k0;
+    apply_split(pend.e, split, nsplit, g.M, 0);
+    pend.m = g.M;
+    pend.n = g.N;
+    pend.row0 = m0 + (wave >> 1) * 128 + (lane & 15);
+    pend.col0 = n0 + (wave & 1) * 128 + 8 * (lane >> 4);
+    return true;
+  };
   constexpr int S = Wide::kOpBytes;
-  wide_core<T, AMN, BMN>(acc, lds_raw, lds_raw + S, lds_raw + 2 * S, lds_raw + 3 * S, pa, pb, g.lda, g.ldb,
-                         min(Wide::BM, g.M - m0), min(Wide::BN, g.N - n0), KT, g.ka - (int)k0, g.kb - (int)k0, wave,
-                         (int)threadIdx.x & 63);
-  Epi e = epi;
-  apply_split(e, split, nsplit, g.M, 0);
-  wide_epilogue(acc, lds_raw, m0, n0, g, e);
+  wide_core<T, AMN, BMN>(
+      lds_raw, lds_raw + S, lds_raw + 2 * S, lds_raw + 3 * S, A, B, g.lda, g.ldb, wave, lane,
+      [&](WideTile& t) {
+        out = pend;
+        return next(t);
+      },
+      [&]() { out.load(0); }, [&](f32x4_t(&acc)[8][8]) { out.store(acc); });
 }
 
 }  // namespace gemm
