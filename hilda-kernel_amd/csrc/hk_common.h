@@ -105,6 +105,23 @@ __device__ __forceinline__ void store_pack(T* p, const Pack<T, VEC>& r) {
   }
 }
 
+// The 16-byte forms at element alignment: rows of an odd length. gfx950 moves
+// an unaligned dwordx4 as one instruction (one cache line more a wave).
+typedef u32x4 any_u32x4 __attribute__((aligned(2)));
+template <typename T, int VEC>
+__device__ __forceinline__ Pack<T, VEC> load_pack_any(const T* p) {
+  static_assert(sizeof(T) * VEC == 16, "16-byte packs");
+  const u32x4 v = *reinterpret_cast<const any_u32x4*>(p);
+  Pack<T, VEC> r;
+  r.w[0] = v.x; r.w[1] = v.y; r.w[2] = v.z; r.w[3] = v.w;
+  return r;
+}
+template <typename T, int VEC>
+__device__ __forceinline__ void store_pack_nt_any(T* p, const Pack<T, VEC>& r) {
+  static_assert(sizeof(T) * VEC == 16, "16-byte packs");
+  __builtin_nontemporal_store(u32x4{r.w[0], r.w[1], r.w[2], r.w[3]}, reinterpret_cast<any_u32x4*>(p));
+}
+
 // Streaming store for outputs that are not re-read by this kernel.
 template <typename T, int VEC>
 __device__ __forceinline__ void store_pack_nt(T* p, const Pack<T, VEC>& r) {

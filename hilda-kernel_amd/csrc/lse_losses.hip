@@ -41,7 +41,7 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
   return r;
 }
 
-template <typename T, int VEC, int NCH, int BLOCK, int NFULL = 0>
+template <typename T, int VEC, int NCH, int BLOCK, int NFULL = 0, bool RAG = false>
 struct RowRegs {
   static_assert(NFULL <= NCH, "full vectors");
   Pack<T, VEC> v[NCH];
@@ -59,7 +59,32 @@ struct RowRegs {
   // reduction's tests stay scalar branches even where they always pass: each
   // vector's work then stays a block of its own, which keeps the compiler
   // from overlapping the vectors' temporaries (and spilling).
+  //
+  // RAG: rows at element alignment whose length is any n >= VEC. The lane of
+  // the row's last, incomplete vector takes the row's last VEC elements
+  // instead: those that the lane before it also holds count once (mask_tail)
+  // and are stored twice, with the same values. (Such rows took one element a
+  // lane, in two passes over memory: the GRPO call on [8, 513, 50257] bf16,
+  // two thirds of the rows live, took 325 us and takes 196. Bound by HBM, with
+  // the odd rows' extra cache line a wave.)
   static constexpr int kSpan = BLOCK * VEC;
+  __device__ __forceinline__ static Pack<T, VEC> get(const T* p) {
+    if constexpr (RAG) return load_pack_any<T, VEC>(p);
+    else return load_pack<T, VEC>(p);
+  }
+  __device__ __forceinline__ static void put(T* p, const Pack<T, VEC>& x) {
+    if constexpr (RAG) store_pack_nt_any<T, VEC>(p, x);
+    else store_pack_nt<T, VEC>(p, x);
+  }
+  // the column, from vector j's first, of a lane's elements in a partial vector of lim columns (lanes past the
+  // row end: in-bounds ones), and how far that is left of the lane's own column
+  __device__ __forceinline__ static int part_col(int tc, int lim) {
+    const int own = tc < lim ? tc : 0;
+    return RAG ? min(own, lim - VEC) : own;
+  }
+  __device__ __forceinline__ static int part_shift(int tc, int lim) {
+    return RAG && tc < lim ? max(0, tc - (lim - VEC)) : 0;
+  }
   __device__ __forceinline__ static int lane_col() { return (int)threadIdx.x * VEC; }
   // element offset of vector j for a lane at column tc, as an unsigned 32-bit
   // value: the address is then one 64-bit base plus a zero-extended VGPR offset
@@ -78,9 +103,9 @@ struct RowRegs {
     for (int j = 0; j < NCH; ++j) {
       const int lim = n - j * kSpan;  // uniform
       if (j < NFULL || lim >= kSpan) {
-        v[j] = load_pack<T, VEC>(row + off(j, tc));
+        v[j] = get(row + off(j, tc));
       } else if (lim > 0) {
-        v[j] = load_pack<T, VEC>(row + off(j, tc < lim ? tc : 0));  // in-bounds address
+        v[j] = get(row + off(j, part_col(tc, lim)));  // in-bounds address
       } else {
         v[j] = ninf;  // defined on every path, so no value flows in from the previous row
       }
@@ -91,9 +116,9 @@ struct RowRegs {
   __device__ __forceinline__ static void mask_tail(int j, int n, float (&x)[VEC]) {
     const int lim = n - j * kSpan;  // uniform
     if (lim < kSpan) {
-      const bool in_row = lane_col() < lim;
+      const int tc = lane_col(), first = tc < lim ? part_shift(tc, lim) : VEC;
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) x[e] = in_row ? x[e] : -INFINITY;
+      for (int e = 0; e < VEC; ++e) x[e] = (RAG ? e >= first : tc < lim) ? x[e] : -INFINITY;
     }
   }
 
@@ -115,7 +140,8 @@ struct RowRegs {
   __device__ __forceinline__ void reduce_lane(int n, float c, int target, float* m_out, float* s_out,
                                               float* xt_out = nullptr) {
     const int jt = target >= 0 ? target / kSpan : -1;  // uniform
-    const int rel = target - jt * kSpan - lane_col();  // in [0, VEC) in the owning lane only
+    // in [0, VEC) in the owning lane only (RAG: or where the element is masked)
+    const int rel = target - jt * kSpan - lane_col() + part_shift(lane_col(), n - jt * kSpan);
     float m = -INFINITY, xt = 0.f;
 #pragma unroll
     for (int j = 0; j < NCH; ++j) {
@@ -164,6 +190,11 @@ struct RowRegs {
   __device__ __forceinline__ static bool owns_target(int target) {
     return target >= 0 && (target % kSpan) / VEC == (int)threadIdx.x;
   }
+  // Whether this lane's stores cover column `target`, so that it has to store that element after them.
+  __device__ __forceinline__ static bool covers_target(int target, int n) {
+    return owns_target(target) ||
+           (RAG && n % VEC != 0 && target >= n - VEC && ((n - 1) % kSpan) / VEC == (int)threadIdx.x);
+  }
 
   // Gradient of the row, p_j * g = 2^(x_j*c - lse2) * g computed in fp32 and
   // rounded once to T (the arithmetic of kernels/cross_entropy.py:159-166),
@@ -187,14 +218,15 @@ struct RowRegs {
         unpack(v[j], x);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) x[e] = exp2_fast(fmaf(x[e], c, -lse2)) * g;
-        if (j < NFULL || lim >= kSpan || tc < lim) store_pack_nt<T, VEC>(out + off(j, tc), pack<T, VEC>(x));
+        if (j < NFULL || lim >= kSpan) put(out + off(j, tc), pack<T, VEC>(x));
+        else if (tc < lim) put(out + off(j, part_col(tc, lim)), pack<T, VEC>(x));
       }
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int j = 0; j < NCH; ++j) {
       const int lim = n - j * kSpan;  // uniform
-      if (j < NFULL || lim > 0) v[j] = load_pack<T, VEC>(next + off(j, lim >= kSpan || tc < lim ? tc : 0));  // see load()
+      if (j < NFULL || lim > 0) v[j] = get(next + off(j, j < NFULL || lim >= kSpan ? tc : part_col(tc, lim)));  // see load()
     }
   }
 };
@@ -209,11 +241,13 @@ __device__ __forceinline__ int row_len(int64_t v) {
   return n;
 }
 
-template <typename T, int VEC, int BLOCK>
+template <typename T, int VEC, int BLOCK, bool RAG = false>
 __device__ __forceinline__ void fill_row(T* __restrict__ out, int n, float value) {
   const Pack<T, VEC> z = splat_pack<T, VEC>(value);
-  for (int col = (int)threadIdx.x * VEC; col < n; col += BLOCK * VEC)
-    store_pack_nt<T, VEC>(out + col, z);
+  for (int col = (int)threadIdx.x * VEC; col < n; col += BLOCK * VEC) {
+    if constexpr (RAG) store_pack_nt_any<T, VEC>(out + min(col, n - VEC), z);
+    else store_pack_nt<T, VEC>(out + col, z);
+  }
 }
 
 // (m, s) <- merge with (m2, s2), where s is a sum of 2^(v - m)
@@ -453,7 +487,7 @@ __device__ __forceinline__ float ce_scale(const CeArgs& a) {
 // Training forward: loss_r = (lse - x_t) * s and dlogits = (softmax - onehot) * s
 // (kernels/cross_entropy.py:114-166). Ignored rows: loss 0 and a zero row,
 // never read.
-template <typename T, int VEC, int NCH, int BLOCK, bool RESIDENT>
+template <typename T, int VEC, int NCH, int BLOCK, bool RESIDENT, bool RAG = false>
 __global__ __launch_bounds__(BLOCK) void ce_fwd_grad_kernel(T* dlogits, const T* logits, CeArgs a) {
   // dlogits may alias logits (in-place use): every element is read before the
   // same thread overwrites it, and a row's stores are issued before the next
@@ -464,14 +498,14 @@ __global__ __launch_bounds__(BLOCK) void ce_fwd_grad_kernel(T* dlogits, const T*
   const int64_t G = gridDim.x;
   auto is_live = [&](int64_t t) { return !(a.has_ignore && t == a.ignore_index) && t >= 0 && t < a.V; };
   if constexpr (RESIDENT) {
-    using Regs = RowRegs<T, VEC, NCH, BLOCK, full_vectors(NCH, BLOCK)>;
+    using Regs = RowRegs<T, VEC, NCH, BLOCK, full_vectors(NCH, BLOCK), RAG>;
     const int n = row_len(a.V);
     // dead rows (ignored or out of range) first: a zero (NaN) row, never read
     for (int64_t row = blockIdx.x; row < a.rows; row += G) {
       const int64_t t = a.targets[row];
       if (!is_live(t)) {
         const bool ignored = a.has_ignore && t == a.ignore_index;
-        fill_row<T, VEC, BLOCK>(dlogits + row * a.ld_out, n, ignored ? 0.f : NAN);
+        fill_row<T, VEC, BLOCK, RAG>(dlogits + row * a.ld_out, n, ignored ? 0.f : NAN);
         if (threadIdx.x == 0) a.loss_rows[row] = ignored ? 0.f : NAN;
       }
     }
@@ -523,7 +557,7 @@ __global__ __launch_bounds__(BLOCK) void ce_fwd_grad_kernel(T* dlogits, const T*
       r.store_prob_grad_then_load(out, n, kLog2e, lse2, gscale, src);
       // the target element: (p_t - 1) * g = -(1 - p_t) * g, stored after (and
       // over) the vector store of the same thread
-      if (Regs::owns_target(t)) out[t] = from_f32<T>(-rest * gscale);
+      if (Regs::covers_target(t, n)) out[t] = from_f32<T>(-rest * gscale);
       if (threadIdx.x == 0) a.loss_rows[row] = (lse2 * kLn2 - X) * scale;
       if (next.q >= nq) break;
       cur = next;
@@ -897,7 +931,7 @@ __device__ __forceinline__ GrpoOut grpo_terms(const GrpoHot& a, const GrpoTok& t
   return GrpoOut{lse, loss, kl, clipped ? 1.f : 0.f};
 }
 
-template <typename T, int VEC, int NCH, int BLOCK, bool RESIDENT, bool GRAD>
+template <typename T, int VEC, int NCH, int BLOCK, bool RESIDENT, bool GRAD, bool RAG = false>
 __global__ __launch_bounds__(BLOCK) void grpo_kernel(T* dlogits, const T* logits, GrpoHot a) {
   // dlogits may alias logits (FusedLinear-GRPO writes the gradient over the
   // chunk's logits): every element is read by the thread that later
@@ -926,7 +960,7 @@ __global__ __launch_bounds__(BLOCK) void grpo_kernel(T* dlogits, const T* logits
   for (int64_t row = blockIdx.x; row < rows; row += G) {
     GrpoTok tk{};
     if (!live(row, &tk)) {
-      if constexpr (GRAD) fill_row<T, VEC, BLOCK>(dlogits + row * a.ld, (int)a.W, 0.f);
+      if constexpr (GRAD) fill_row<T, VEC, BLOCK, RAG>(dlogits + row * a.ld, (int)a.W, 0.f);
       const int64_t g = pos(row), b = g / (a.L + 1), l = g - b * (a.L + 1);
       if (l < a.L && threadIdx.x == 0) a.out[b * a.L + l] = GrpoOut{0.f, 0.f, 0.f, 0.f};
     }
@@ -941,7 +975,7 @@ __global__ __launch_bounds__(BLOCK) void grpo_kernel(T* dlogits, const T* logits
     // with the gradient stores, the per-row records are scalar loads (the
     // search for the row after next runs at the end of the iteration) and the
     // id logit comes out of the registers through the block exchange.
-    using Regs = RowRegs<T, VEC, NCH, BLOCK, full_vectors(NCH, BLOCK)>;
+    using Regs = RowRegs<T, VEC, NCH, BLOCK, full_vectors(NCH, BLOCK), RAG>;
     // (the token's id rides along; the rest of its record is loaded again
     // when the row starts, in time for the loss terms after the exchange)
     struct LiveRow {
@@ -996,7 +1030,7 @@ __global__ __launch_bounds__(BLOCK) void grpo_kernel(T* dlogits, const T* logits
         T* out = dlogits + row * a.ld;
         r.store_prob_grad_then_load(out, n, c, lse2, g, src);
         // the id element: (p_id - 1) * g = -(1 - p_id) * g (see reduce_lane)
-        if (Regs::owns_target(id)) out[id] = from_f32<T>(-rest * g);
+        if (Regs::covers_target(id, n)) out[id] = from_f32<T>(-rest * g);
       }
       if (threadIdx.x == 0) a.out[cur.tok_i] = res;
       if (next.row >= rows) break;
@@ -1018,7 +1052,7 @@ __global__ __launch_bounds__(BLOCK) void grpo_kernel(T* dlogits, const T* logits
       const float xid = tk.id >= 0 ? to_f32<T>(in[tk.id]) : 0.f;
       float lse2, rest = 0.f;
       if constexpr (RESIDENT) {  // (forward only: the gradient form's arithmetic, see lse_rows_resident)
-        RowRegs<T, VEC, NCH, BLOCK> r;
+        RowRegs<T, VEC, NCH, BLOCK, 0, RAG> r;
         r.load(in, n);
         float m, s, M, S;
         r.reduce_lane(n, c, tk.id, &m, &s);
@@ -1239,14 +1273,19 @@ struct RowCfg {
   int block;
   int nch;  // 0: streaming
   int vec;  // elements per vector
+  bool rag = false;  // register-resident, rows at element alignment (RowRegs' RAG)
 };
 
-RowCfg choose_row_cfg(int64_t V, int esize, bool vec_ok) {
-  RowCfg c{1024, 0, vec_ok ? 16 / esize : 1};
-  if (!vec_ok) return c;
-  const int64_t nv = V / c.vec;
+// rag_ok: the caller's kernel has the RAG forms (the gradient kernels and GRPO's forward: they hold the row for a
+// second use, which the one-element-a-lane loop reads again). Rows shorter than a vector, or longer than every form,
+// keep one element a lane.
+RowCfg choose_row_cfg(int64_t V, int esize, bool vec_ok, bool rag_ok = false) {
+  const int vec = 16 / esize;
+  RowCfg c{1024, 0, vec_ok ? vec : 1};
+  if (!vec_ok && (!rag_ok || V < vec)) return c;
+  const int64_t nv = cdiv(V, vec);
   for (const RowForm& f : kRowForms)
-    if (nv <= (int64_t)f.block * f.nch) return RowCfg{f.block, f.nch, c.vec};
+    if (nv <= (int64_t)f.block * f.nch) return RowCfg{f.block, f.nch, vec, !vec_ok};
   return c;
 }
 
@@ -1398,7 +1437,7 @@ int grpo_rows_launch(void* dlogits, const void* logits, int64_t row0, int64_t nr
   const int es = esize(dtype);
   const bool vec_ok = width % (16 / es) == 0 && (ld * es) % 16 == 0 && aligned_to(logits, 16) &&
                       (!dlogits || aligned_to(dlogits, 16));
-  const RowCfg cfg = choose_row_cfg(width, es, vec_ok);
+  const RowCfg cfg = choose_row_cfg(width, es, vec_ok, true);
   return dispatch_t(dtype, [&](auto tt) {
     using T = typename decltype(tt)::type;
     return dispatch_cfg(cfg, [&](auto blk, auto nch) {
@@ -1417,6 +1456,7 @@ int grpo_rows_launch(void* dlogits, const void* logits, int64_t row0, int64_t nr
         } else {
           // the resident form takes its leading full vectors untested (see form_fits)
           if (!form_fits(width, cfg)) return HK_EINVAL;
+          if (cfg.rag) return run(grpo_kernel<T, 16 / sizeof(T), NCH, BLOCK, true, GRAD, true>, BLOCK);
           return run(grpo_kernel<T, 16 / sizeof(T), NCH, BLOCK, true, GRAD>, BLOCK);
         }
       };
@@ -1546,7 +1586,7 @@ int ce_rows_launch(void* dlogits, float* loss_rows, const void* logits, const in
   const int vec = 16 / es;
   const bool vec_ok = V % vec == 0 && aligned_to(logits, 16) && aligned_to(dlogits, 16) && (ld_in * es) % 16 == 0 &&
                       (ld_out * es) % 16 == 0;
-  const RowCfg cfg = choose_row_cfg(V, es, vec_ok);
+  const RowCfg cfg = choose_row_cfg(V, es, vec_ok, true);
   return dispatch_t(dtype, [&](auto tt) {
     using T = typename decltype(tt)::type;
     return dispatch_cfg(cfg, [&](auto blk, auto nch) {
@@ -1563,6 +1603,7 @@ int ce_rows_launch(void* dlogits, float* loss_rows, const void* logits, const in
         return run(ce_fwd_grad_kernel<T, 16 / sizeof(T), 1, BLOCK, false>, BLOCK);
       } else {
         if (!form_fits(V, cfg)) return HK_EINVAL;
+        if (cfg.rag) return run(ce_fwd_grad_kernel<T, 16 / sizeof(T), NCH, BLOCK, true, true>, BLOCK);
         return run(ce_fwd_grad_kernel<T, 16 / sizeof(T), NCH, BLOCK, true>, BLOCK);
       }
     });
