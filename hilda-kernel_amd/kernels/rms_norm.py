@@ -17,7 +17,7 @@ from . import _lib
 
 def _rows_view(t: torch.Tensor, hidden: int) -> torch.Tensor:
     """2-D [rows, hidden] view with unit column stride (copies only if needed)."""
-    t2 = t.reshape(-1, hidden)
+    t2 = t if t.dim() == 2 and hidden and t.shape[1] == hidden else t.reshape(-1, hidden)
     if t2.stride(-1) != 1 or (t2.shape[0] > 1 and t2.stride(0) < hidden):
         t2 = t2.contiguous()
     return t2

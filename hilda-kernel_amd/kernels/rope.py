@@ -36,31 +36,32 @@ def _launch(x_in, x_out, cos, sin, inverse):
 
 def _launch_qk(q_in, q_out, k_in, k_out, cos, sin, inverse):
     """q and k in one launch when they share batch, positions, head_dim and dtype."""
+    # shapes and strides are read once each: as properties and single strides they were 3 us of host time a call
     bsz, hq, seq_len, hd = q_in.shape
-    same = (k_in.shape[0] == bsz and k_in.shape[2] == seq_len and k_in.shape[3] == hd and k_in.dtype == q_in.dtype
-            and q_in.stride(-1) == 1 and k_in.stride(-1) == 1)
+    kb, hk, kt, kd = k_in.shape
+    qi, ki = q_in.stride(), k_in.stride()
+    same = kb == bsz and kt == seq_len and kd == hd and k_in.dtype == q_in.dtype and qi[3] == 1 and ki[3] == 1
     if not same or q_in.numel() == 0 or k_in.numel() == 0:
         _launch(q_in, q_out, cos, sin, inverse)
         _launch(k_in, k_out, cos, sin, inverse)
         return
-    assert q_out.stride(-1) == 1 and k_out.stride(-1) == 1
-    assert cos.shape == sin.shape and cos.dim() == 3 and cos.shape[-1] == hd // 2, \
-        f"cos/sin must be (1 or bsz, seq, head_dim/2); got {tuple(cos.shape)}"
-    assert cos.shape[1] >= seq_len, f"cos/sin cover {cos.shape[1]} positions, need {seq_len}"
-    assert cos.shape[0] in (1, bsz)
-    assert cos.dtype == sin.dtype and cos.stride() == sin.stride()
-    _lib.call("hk_rope_qk", q_out.data_ptr(), q_in.data_ptr(), hq,
-              q_in.stride(0), q_in.stride(1), q_in.stride(2), q_out.stride(0), q_out.stride(1), q_out.stride(2),
-              k_out.data_ptr(), k_in.data_ptr(), k_in.shape[1],
-              k_in.stride(0), k_in.stride(1), k_in.stride(2), k_out.stride(0), k_out.stride(1), k_out.stride(2),
-              cos.data_ptr(), sin.data_ptr(), bsz, seq_len, hd, cos.shape[0], cos.stride(0), cos.stride(1),
+    qo, ko, cst, csh = q_out.stride(), k_out.stride(), cos.stride(), cos.shape
+    assert qo[3] == 1 and ko[3] == 1
+    assert csh == sin.shape and len(csh) == 3 and csh[2] == hd // 2, \
+        f"cos/sin must be (1 or bsz, seq, head_dim/2); got {tuple(csh)}"
+    assert csh[1] >= seq_len, f"cos/sin cover {csh[1]} positions, need {seq_len}"
+    assert csh[0] in (1, bsz)
+    assert cos.dtype == sin.dtype and cst == sin.stride()
+    _lib.call("hk_rope_qk", q_out.data_ptr(), q_in.data_ptr(), hq, qi[0], qi[1], qi[2], qo[0], qo[1], qo[2],
+              k_out.data_ptr(), k_in.data_ptr(), hk, ki[0], ki[1], ki[2], ko[0], ko[1], ko[2],
+              cos.data_ptr(), sin.data_ptr(), bsz, seq_len, hd, csh[0], cst[0], cst[1],
               _lib.dtype_code(q_in), _lib.dtype_code(cos), int(inverse), _lib.stream_of(q_in.device))
 
 
 def _tables(cos, sin):
     if cos.stride(-1) != 1:
         cos = cos.contiguous()
-    if sin.stride(-1) != 1 or sin.stride() != cos.stride():
+    if sin.stride() != cos.stride():  # (cos' last stride is 1)
         sin = sin.contiguous()
         cos = cos.contiguous()
     return cos, sin
