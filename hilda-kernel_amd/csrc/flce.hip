@@ -1480,8 +1480,9 @@ namespace {
 // reference to follow): twice the bytes of the weight (the size of its
 // gradient, which the op allocates anyway, twice over). Below it the plans
 // fall back to short chunks, whose dW GEMM re-reads and rewrites the whole
-// weight gradient every chunk: at B 16, L+1 1024, H 4096, V 151936 bf16 95 ms
-// with a 150 MB plan, 44 ms at the floor, 36 ms with no limit.
+// weight gradient every chunk: at B 16, L+1 1024, H 4096, V 151936 bf16, 9444
+// live tokens, 100 ms with a 150 MB plan, 31 ms at the floor, 28 ms with no
+// limit.
 size_t weight_pair_bytes(int64_t V, int64_t H, int es) { return 2 * (size_t)V * (size_t)pad8(H) * (size_t)es; }
 
 // Default-budget floor of FusedLinearJSD: what the reference's chunk loop
@@ -1493,7 +1494,7 @@ size_t weight_pair_bytes(int64_t V, int64_t H, int es) { return 2 * (size_t)V * 
 // it is added into grad_weight. The op's outputs are the reference's, so a
 // workspace within this keeps its peak memory at or below the reference's.
 // (Smaller budgets mean short chunks: BT 8192, H 4096, V 128256 bf16 ran
-// 60 ms at 256 MiB, 38 ms at 1 GiB, 35 ms at 1.5 GiB, 31 ms with no limit.)
+// 55 ms at 256 MiB, 32 ms at 1 GiB, 30 ms at 1.5 GiB, 27 ms with no limit.)
 size_t jsd_reference_bytes(int64_t BT, int64_t H, int64_t V, int es) {
   // the reference's chunk rows, unclamped (fused_linear_jsd.py:133-135), at most BT
   const int64_t per = std::max<int64_t>(1, cdiv(BT, cdiv(V, H)));
