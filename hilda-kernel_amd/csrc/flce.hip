@@ -800,18 +800,24 @@ struct FlPlan {
 
 int dx_bk(int es) { return es == 4 ? gemm::F32Cfg::BK : gemm::DefaultCfg::BK; }
 
-// fp32 partial-sum bytes the dX GEMM of a chunk of up to C rows can need with at
-// most smax splits: the largest splits x rows over the row counts it may be cut to.
-size_t dx_part_bytes(int64_t C, int64_t Hp, int64_t ldl, int bk, int smax) {
-  if (smax <= 1) return 0;
-  size_t best = 0;
-  const int64_t ntn = cdiv(Hp, 256), kt = ldl / bk;
-  for (int64_t mt = 1; mt <= cdiv(C, 256); ++mt) {
-    const int s = gemm::auto_splits((int)(mt * ntn), (int)kt, smax);
-    if (s > 1) best = std::max(best, (size_t)s * (size_t)std::min<int64_t>(C, mt * 256) * Hp * 4);
+// fp32 partial-sum bytes the dX GEMM of a chunk of up to C rows can need with at most smax splits: the largest splits
+// x rows over the row counts it may be cut to. The whole row tiles' part is kept over the chunk sizes of one planning
+// (worked out for each chunk size it was half of the planner's time).
+struct DxPartials {
+  int64_t Hp, kt, ntn;
+  int smax;
+  std::vector<size_t> whole;  // [t]: the most for chunks cut to at most t whole tiles
+
+  DxPartials(int64_t cmax, int64_t hp, int64_t ldl, int bk, int most)
+      : Hp(hp), kt(ldl / bk), ntn(cdiv(hp, 256)), smax(most), whole(1, 0) {
+    for (int64_t t = 1; t <= cmax / 256; ++t) whole.push_back(std::max(whole.back(), of(t, t * 256)));
   }
-  return best;
-}
+  size_t of(int64_t t, int64_t rows) const {
+    const int s = smax > 1 ? gemm::auto_splits((int)(t * ntn), (int)kt, smax) : 1;
+    return s > 1 ? (size_t)s * (size_t)rows * Hp * 4 : 0;
+  }
+  size_t bytes(int64_t C) const { return std::max(whole[C / 256], C % 256 ? of(C / 256 + 1, C) : 0); }
+};
 
 // The workspace layout of one candidate (C rows a chunk, the forms, the split cap and its partials' bytes).
 FlPlan fl_layout(const FlShape& s, int64_t C, bool wt, bool dt, int dw, int smax, size_t pb) {
@@ -896,19 +902,32 @@ FlPlan vt_layout(const FlShape& s, int64_t Vt, int dw) {
   return p;
 }
 
-// Rate of the 16-bit GEMM kernel in any operand layout, alone on the chip (gemm_wide.h), and of streaming passes
-// over memory. (fp32 plans only compare with each other: the same forms at one rate.)
-constexpr double kGemmRate = 1.4e15, kStreamRate = 5.0e12, kLaunch = 5e-6;
+// What the cost of a plan is modelled from: the 16-bit GEMMs' rate, the factor on a GEMM's time for each MN-contiguous
+// operand, whether every dW GEMM reads a transposed X (else only beside a transposed D), and whether the
+// vocabulary-tiled GEMMs' part-filled tiles of rows are charged whole. (fp32 plans only compare with each other: the
+// same forms at one rate.)
+struct CostModel {
+  double gemm, mn;
+  bool xt, whole_tiles;
+};
+// The kernels as they are: one rate in any operand layout, alone on the chip (gemm_wide.h).
+constexpr CostModel kModel{1.4e15, 1.0, false, true};
+// The model that draws the line between fp32 sums and sums in the 16-bit output (see fl_plan). These were the rates of
+// an 8-wave GEMM; they stay when the kernels get faster, because with other rates the line moves: kModel alone gave 138
+// of 91440 calls (FusedLinearCE, JSD and GRPO; H 512-5120, V 8000-151936) 16-bit sums in the place of fp32 ones and
+// 420 more of the roundings they had.
+constexpr CostModel kSumModel{1.25e15, 1.2, true, false};
+constexpr double kStreamRate = 5.0e12, kLaunch = 5e-6;  // streaming passes over memory; a launch
 
 // Modelled time of a vocabulary-tiled candidate: the logits GEMM twice (the
 // log-sum-exp pass, then the gradient pass), the dW and dX GEMMs, idle CUs when
 // a GEMM has fewer than 256 tiles, the row passes' HBM bytes and dX's
 // read-modify-writes.
-double vt_cost(const FlShape& s, const FlPlan& p) {
-  const double Rg = kGemmRate, Rm = kStreamRate, launch = kLaunch;
+double vt_cost(const FlShape& s, const FlPlan& p, const CostModel& m) {
+  const double Rg = m.gemm, Rm = kStreamRate, launch = kLaunch;
   const double es = s.es, BT = (double)s.BT, Hp = (double)p.Hp, V = (double)s.V;
   // (a 256-row tile costs the same whatever part of it is rows)
-  const double F = 2.0 * (double)(cdiv(s.BT, 256) * 256) * Hp * V;
+  const double F = 2.0 * (m.whole_tiles ? (double)(cdiv(s.BT, 256) * 256) : BT) * Hp * V;
   // a GEMM of `tiles` 256x256 tiles takes whole waves of 256 (one workgroup a CU)
   auto fill = [](int64_t tiles) {
     tiles = std::max<int64_t>(tiles, 1);
@@ -920,7 +939,8 @@ double vt_cost(const FlShape& s, const FlPlan& p) {
   if (p.wpad) t += 2.0 * es * V * Hp / Rm;
   if (s.grad) {
     t += F / Rg * fill(tb * tv) + 2.0 * BT * V * es / Rm;
-    t += F / Rg * fill(tv * th) + F / Rg * fill(tb * th);
+    t += F / Rg * fill(tv * th) * m.mn * m.mn;
+    t += F / Rg * fill(tb * th) * m.mn;
     const double nt = (double)p.ntiles;
     t += (p.dw == kDwAcc ? 8.0 * BT * Hp * (nt - 1) : 2.0 * es * BT * Hp * (nt - 1)) / Rm;
     t += p.ntiles * 4 * launch;
@@ -928,14 +948,19 @@ double vt_cost(const FlShape& s, const FlPlan& p) {
   return t;
 }
 
-// Modelled time (seconds) of a candidate: the GEMMs at one rate whatever their
-// operands' layout, tile waste of a short chunk, a dX GEMM that leaves CUs
-// idle, and the HBM bytes of the transposes, the dW read-modify-writes, the
-// split partials and the gathers, plus launches. (BT 2048, H 4096, V 32000:
-// 1.49 ms with W^T, D^T and X^T, 1.43 without D^T and X^T, 1.40 without W^T, 1.34
-// without any.)
-double fl_cost(const FlShape& s, const FlPlan& p) {
-  const double Rg = kGemmRate, Rm = kStreamRate, launch = kLaunch;
+// What a row-chunked candidate is modelled from, the same in every cost model: each GEMM's FLOPs, with tile waste of a
+// short chunk and CUs left idle, and the seconds of the HBM bytes of the transposes, the dW read-modify-writes, the
+// split partials and the gathers, plus launches; X^T apart. (BT 2048, H 4096, V 32000: 1.49 ms with W^T, D^T and X^T,
+// 1.43 without D^T and X^T, 1.40 without W^T, 1.34 without any.)
+struct FlWork {
+  double logits = 0, dx = 0, dw = 0, rest = 0, xt = 0;
+  bool wt, dt;
+  double seconds(const CostModel& m) const {
+    return (logits + dx * (wt ? 1.0 : m.mn) + dw * (dt ? 1.0 : m.mn)) / m.gemm + rest + (dt || m.xt ? xt : 0.0);
+  }
+};
+FlWork fl_work(const FlShape& s, const FlPlan& p) {
+  const double Rm = kStreamRate, launch = kLaunch;
   const double es = s.es, BT = (double)s.BT, Hp = (double)p.Hp, V = (double)s.V;
   const double F = 2.0 * BT * Hp * V;
   // row waste of a chunk's last 256-row tile, and whole waves of 256 workgroups (one a CU)
@@ -945,24 +970,29 @@ double fl_cost(const FlShape& s, const FlPlan& p) {
     return (double)(cdiv(wgs, 256) * 256) / (double)wgs;
   };
   const double nch = (double)p.nch;
-  double t = F / Rg * q * waves(cdiv(p.C, 256) * cdiv(s.V, 256)) + nch * 6 * launch;
-  if (p.gather) t += 2.0 * es * BT * Hp / Rm;
-  if (p.wpad) t += 2.0 * es * V * Hp / Rm;
+  FlWork w;
+  w.wt = p.wt;
+  w.dt = p.dt;
+  w.logits = F * q * waves(cdiv(p.C, 256) * cdiv(s.V, 256));
+  w.rest = nch * 6 * launch;
+  if (p.gather) w.rest += 2.0 * es * BT * Hp / Rm;
+  if (p.wpad) w.rest += 2.0 * es * V * Hp / Rm;
   if (s.grad) {
     const int64_t tiles = cdiv(p.C, 256) * cdiv(p.Hp, 256);
     const int sp = gemm::auto_splits((int)tiles, (int)(p.ldl / dx_bk(s.es)), p.ksplit);
-    t += F / Rg * q * waves(tiles * sp);
-    if (sp > 1) t += nch * 2.0 * sp * (double)p.C * Hp * 4 / Rm;
-    t += F / Rg * waves(cdiv(s.V, 256) * cdiv(p.Hp, 256));
+    w.dx = F * q * waves(tiles * sp);
+    if (sp > 1) w.rest += nch * 2.0 * sp * (double)p.C * Hp * 4 / Rm;
+    w.dw = F * waves(cdiv(s.V, 256) * cdiv(p.Hp, 256));
     double rmw = es * V * Hp;
     if (p.dw == kDwAcc && p.nch > 1) rmw = 8.0 * V * Hp * (nch - 1) + es * V * Hp;
     if (p.dw == kDwOut) rmw = es * V * Hp * (2 * nch - 1);
-    t += rmw / Rm;
-    if (p.wt) t += 2.0 * es * V * Hp / Rm;
-    if (p.dt) t += 2.0 * es * BT * ((double)p.V8 + Hp) / Rm + nch * 2 * launch;
-    t += nch * 2 * launch;
+    w.rest += rmw / Rm;
+    if (p.wt) w.rest += 2.0 * es * V * Hp / Rm;
+    if (p.dt) w.rest += 2.0 * es * BT * (double)p.V8 / Rm;
+    w.rest += nch * 2 * launch;
+    w.xt = 2.0 * es * BT * Hp / Rm + nch * 2 * launch;
   }
-  return t;
+  return w;
 }
 
 // The reference's chunk rule (fused_linear_cross_entropy.py:112-114): chunk
@@ -1032,23 +1062,88 @@ bool forced_form(int* dw, bool* wt, bool* dt, int64_t* vt, bool* bad) {
 constexpr size_t kSmallWorkspace = (size_t)40 << 20;
 
 // A plan that sums dW (and dX) in fp32 is taken over a faster one that sums in
-// the 16-bit output unless it is modelled this much slower. Vocabulary tiles
+// the 16-bit output unless it is modelled this much slower (by kSumModel, see
+// fl_plan; kModel may only move a call towards fp32). Vocabulary tiles
 // wider than 8192 columns, for few rows: their GEMMs have few workgroups, and
 // beyond 1.3 a call got slower (1024 rows, H 1024, V 50257: 1.26 -> 1.41 ms).
 constexpr double kExactSlack = 1.5, kWideTileSlack = 1.3;
 
-// dW summed in fp32 (or computed whole): every form but accumulation in a
-// 16-bit output over several chunks.
-bool exact_dw(const FlShape& s, const FlPlan& p) { return !s.grad || p.dw != kDwOut || p.nch <= 1 || s.es == 4; }
-// (a vocabulary-tiled plan writes dW once; its dX is summed across the tiles in the same ways)
+// A candidate plan: what fl_layout (vt_layout) is called with, and its bytes and modelled seconds.
+struct FlChoice {
+  int64_t C = 0, n = 0;  // rows a chunk and chunks, or columns a tile and tiles
+  bool vtile = false, wt = false, dt = false;
+  int dw = kDwOut, smax = 1;
+  size_t part = 0, total = 0;
+  double cost = 0;
+};
+
+// How often a gradient is rounded to 16 bits between two partial sums: dW in the output over row chunks, dX in the
+// output over vocabulary tiles.
+struct Roundings {
+  int64_t dw, dx;
+};
+Roundings roundings(const FlShape& s, const FlChoice& c) {
+  const int64_t r = s.grad && s.es != 4 && c.dw == kDwOut ? std::max<int64_t>(c.n - 1, 0) : 0;
+  return c.vtile ? Roundings{0, r} : Roundings{r, 0};
+}
+bool exact_sums(const FlShape& s, const FlChoice& c) {
+  const Roundings r = roundings(s, c);
+  return r.dw == 0 && r.dx == 0;
+}
+
+// The choice among candidates of one cost model: the fastest whose sums are in fp32, unless the fastest of all is
+// modelled more than kExactSlack times faster (kWideTileSlack: see there). fp16 inputs compare with the fastest that
+// does not sum dW in the fp16 output over several chunks, where one fits: gradients scaled by 1/n sit in fp16's
+// subnormal range there, where each rounding costs percent-level error (the vocabulary-tiled plan sums dX unscaled,
+// which stays in the normal range).
+struct FlPick {
+  const FlShape& s;
+  bool found = false, found_safe = false;
+  bool found_ex[2] = {false, false};  // tiles of at most 8192 columns and row chunks; wider tiles
+  FlChoice best, best_ex[2], best_safe;
+
+  void consider(const FlChoice& c) {
+    auto better = [&](const FlChoice& a, const FlChoice& b) {
+      return a.cost < b.cost || (a.cost == b.cost && a.total < b.total);
+    };
+    if (!found || better(c, best)) {
+      best = c;
+      found = true;
+    }
+    const int wide = c.vtile && c.C > 8192;
+    const bool ex = exact_sums(s, c);
+    if (ex && (!found_ex[wide] || better(c, best_ex[wide]))) {
+      best_ex[wide] = c;
+      found_ex[wide] = true;
+    }
+    const bool risky = s.f16 && !c.vtile && !ex;
+    if (!risky && (!found_safe || better(c, best_safe))) {
+      best_safe = c;
+      found_safe = true;
+    }
+  }
+  const FlChoice& take() const {
+    const FlChoice& fast = s.f16 && found_safe ? best_safe : best;
+    const FlChoice* r = nullptr;
+    for (int wide = 0; wide < 2; ++wide) {
+      const FlChoice& e = best_ex[wide];
+      if (found_ex[wide] && e.cost <= (wide ? kWideTileSlack : kExactSlack) * fast.cost && (!r || e.cost < r->cost))
+        r = &e;
+    }
+    return r ? *r : fast;
+  }
+};
 
 // The plan for a byte budget: budget == 0 the default (at most the larger of
 // kSmallWorkspace and what the reference's chunk costs in the leanest form),
-// budget < 0 unlimited, else at most `budget` bytes. Within the budget: the
-// fastest candidate by fl_cost (vt_cost) whose sums are in fp32, unless the
-// fastest of all, which accumulates in the 16-bit output (the reference's
-// arithmetic, fused_linear_cross_entropy.py:161), is modelled more than
-// kExactSlack times faster. HK_EINVAL when nothing fits.
+// budget < 0 unlimited, else at most `budget` bytes. HK_EINVAL when nothing
+// fits.
+//
+// Two models choose. kSumModel, over the forms it prices (tiles of at most 8192
+// columns, X^T in every row-chunked form), makes the choice FlPick describes: it
+// says how often dW and dX may be rounded between partial sums (the reference's
+// own dW is rounded per chunk, fused_linear_cross_entropy.py:161). kModel then
+// chooses in the same way among all forms that round no gradient more often.
 int fl_plan(const FlShape& s, int64_t budget, FlPlan* out) {
   int f_dw = 0;
   int64_t f_vt = 0;
@@ -1062,68 +1157,57 @@ int fl_plan(const FlShape& s, int64_t budget, FlPlan* out) {
     const bool mn_ok = s.es == 2;
     return fl_layout(s, C, !mn_ok, !mn_ok, kDwOut, 1, 0);
   };
+  // bytes of X^T, which kSumModel's row-chunked forms hold beside an untransposed D too
+  auto xt_bytes = [&](const FlPlan& p) {
+    return s.grad && !p.dt ? align256((size_t)p.Hp * ld_t(p.dw == kDwDefer ? s.BT : p.C) * s.es) : 0;
+  };
   size_t cap;
   if (budget == 0) {
     const int64_t C0 = std::min<int64_t>(cmax, ref_chunk(s.BT, s.H, s.V));
     // the reference's chunk logits, the gathered rows and as much again, and an
     // eighth of the chunk's bytes for the dX GEMM's split partials
     const FlPlan b = lean(C0);
-    const size_t rows = s.grad && !b.dt ? (size_t)b.Hp * ld_t(C0) * s.es : 0;
-    cap = std::max({kSmallWorkspace, s.default_floor, b.total + rows + (size_t)C0 * pad64(s.V) * s.es / 8});
+    cap = std::max({kSmallWorkspace, s.default_floor, b.total + xt_bytes(b) + (size_t)C0 * pad64(s.V) * s.es / 8});
   } else {
     cap = budget < 0 ? SIZE_MAX : (size_t)budget;
   }
-  // Without a limit a FusedLinearCE call of several chunks keeps its documented plan: W^T, every chunk's D^T and
-  // one dW GEMM, with the workspace callers size for it (C5: 39.0 ms; W, D and X read MN-contiguous with an
-  // fp32 dW accumulator 38.4 ms, W alone MN-contiguous 38.2). Small hidden sizes, whose accumulator is cheap,
-  // were and stay the model's choice (16384 rows, H 1024, V 32000: 3.53 ms materialised, 3.15 accumulated).
-  const bool materialise = budget < 0 && s.ce && s.grad && !forced && s.BT > cmax && (s.H >= 2048 || s.chunk_cap > 0);
-  // the fastest candidate overall, the fastest whose dW (and dX) are summed in fp32, and (fp16 inputs) the
-  // fastest that does not sum dW in the fp16 output over several chunks: gradients scaled by 1/n sit in
-  // fp16's subnormal range there, where each rounding costs percent-level error (the vocabulary-tiled plan
-  // sums dX unscaled, which stays in the normal range)
-  bool found = false, found_safe = false;
-  bool found_ex[2] = {false, false};  // tiles of at most 8192 columns and row chunks; wider tiles
-  FlPlan best, best_ex[2], best_safe;
-  auto consider = [&](const FlPlan& p) {
-    auto better = [&](const FlPlan& a, const FlPlan& b) {
-      return a.cost < b.cost || (a.cost == b.cost && a.total < b.total);
-    };
-    if (!found || better(p, best)) {
-      best = p;
-      found = true;
-    }
-    const int wide = p.vtile && p.Vt > 8192;
-    if (exact_dw(s, p) && (!found_ex[wide] || better(p, best_ex[wide]))) {
-      best_ex[wide] = p;
-      found_ex[wide] = true;
-    }
-    const bool risky = s.f16 && !p.vtile && !exact_dw(s, p);
-    if (!risky && (!found_safe || better(p, best_safe))) {
-      best_safe = p;
-      found_safe = true;
-    }
-  };
+  FlPick sum{s};
+  std::vector<FlChoice> all;
+  all.reserve(1024);
   std::vector<int64_t> cs;
   for (int64_t C = cmax; C >= 8; C = (C > 64 ? (C - 1) / 64 * 64 : C / 2 & ~(int64_t)7)) {
     cs.push_back(C);
     if (C <= 8) break;
   }
+  std::vector<DxPartials> splits;  // split caps from the most down
+  for (int sm = smax_full; sm >= 1; sm = sm > 1 ? sm / 2 : 0)
+    splits.emplace_back(cmax, pad8(s.H), pad64(s.V), dx_bk(s.es), sm);
   for (int64_t C : cs) {
     const int64_t nch = s.BT > 0 ? cdiv(s.BT, C) : 0;
-    size_t part[4] = {0, 0, 0, 0};  // the partials' bytes at each split cap below
-    if (s.grad)
-      for (int sm = smax_full, i = 0; sm >= 1; sm = sm > 1 ? sm / 2 : 0, ++i)
-        part[i] = dx_part_bytes(C, pad8(s.H), pad64(s.V), dx_bk(s.es), sm);
     fl_forms(s, nch, [&](bool wt, bool dt, int dw) {
       if (forced && (f_vt > 0 || dw != f_dw || wt != f_wt || dt != f_dt)) return;
-      if (materialise && !(wt && dt && dw == kDwDefer)) return;
-      for (int sm = smax_full, i = 0; sm >= 1; sm = sm > 1 ? sm / 2 : 0, ++i) {
-        FlPlan p = fl_layout(s, C, wt, dt, dw, sm, part[i]);
-        if (p.total > cap) continue;
-        p.cost = fl_cost(s, p);
-        consider(p);
-        break;  // fewer splits only if more do not fit
+      FlPlan p = fl_layout(s, C, wt, dt, dw, 1, 0);
+      const size_t xt = xt_bytes(p);
+      bool model = true, rule = !forced;  // which still look for a split cap that fits
+      for (const DxPartials& sp : splits) {
+        const size_t part = s.grad ? sp.bytes(C) : 0;
+        const size_t total = p.total + align256(part);
+        if (total > cap) continue;
+        p.ksplit = part ? sp.smax : 1;
+        FlChoice c{C, nch, false, wt, dt, dw, sp.smax, part, total, 0};
+        const FlWork w = fl_work(s, p);
+        if (model) {
+          c.cost = w.seconds(kModel);
+          all.push_back(c);
+          model = false;  // fewer splits only if more do not fit
+        }
+        if (rule && total + xt <= cap) {
+          c.total = total + xt;
+          c.cost = w.seconds(kSumModel);
+          sum.consider(c);
+          rule = false;
+        }
+        if (!model && !rule) break;
       }
     });
   }
@@ -1131,34 +1215,48 @@ int fl_plan(const FlShape& s, int64_t budget, FlPlan* out) {
     // tiles of up to the whole vocabulary (above 8192 columns in steps of 2048): few rows need wide tiles to
     // fill the chip (500 rows of V 128256: a GEMM of 8192 columns has 64 workgroups)
     const int64_t vmax = (s.V + 255) / 256 * 256;
-    for (int64_t Vt = vmax; Vt >= 256 && !materialise; Vt = Vt > 8192 ? std::max<int64_t>(8192, (Vt - 1) / 2048 * 2048) : Vt - 256)
+    for (int64_t Vt = vmax; Vt >= 256; Vt = Vt > 8192 ? std::max<int64_t>(8192, (Vt - 1) / 2048 * 2048) : Vt - 256)
       for (int dw : {kDwAcc, kDwOut}) {
         if (forced && (Vt != f_vt || dw != f_dw)) continue;
-        FlPlan p = vt_layout(s, Vt, dw);
+        const FlPlan p = vt_layout(s, Vt, dw);
         if (p.total > cap) continue;
-        p.cost = vt_cost(s, p);
-        consider(p);
+        FlChoice c{Vt, p.ntiles, true, false, false, dw, 1, 0, p.total, vt_cost(s, p, kModel)};
+        all.push_back(c);
+        if (forced || Vt > 8192) continue;
+        c.cost = vt_cost(s, p, kSumModel);
+        sum.consider(c);
       }
   }
-  if (!found && forced) {
+  if (all.empty() && forced) {
     set_error("HILDA_FL_FORM: the forced form does not apply to this call (dtype, chunk count or budget)");
     return HK_EINVAL;
   }
-  if (!found) {
+  if (all.empty()) {
     const FlPlan small = lean(cs.back());
     set_error("workspace budget %lld bytes is below the smallest plan (%zu bytes)", (long long)budget, small.total);
     return HK_EINVAL;
   }
-  // fp32 sums unless they cost more than half as much time again as the fastest plan (fp16: the fastest
-  // plan without fp16 dW sums over chunks, when one fits)
-  const FlPlan& fast = s.f16 && found_safe ? best_safe : best;
-  const FlPlan* take = nullptr;
-  for (int wide = 0; wide < 2; ++wide) {
-    const FlPlan& e = best_ex[wide];
-    if (found_ex[wide] && e.cost <= (wide ? kWideTileSlack : kExactSlack) * fast.cost && (!take || e.cost < take->cost))
-      take = &e;
+  FlPick pick{s};
+  if (sum.found) {
+    const FlChoice& r = sum.take();
+    const Roundings rr = roundings(s, r);
+    // Without a limit a FusedLinearCE call of several chunks keeps its documented plan: W^T, every chunk's D^T and
+    // one dW GEMM, with the workspace callers size for it (C5: 39.0 ms; W, D and X read MN-contiguous with an
+    // fp32 dW accumulator 38.4 ms, W alone MN-contiguous 38.2). Small hidden sizes, whose accumulator is cheap,
+    // were and stay the model's choice (16384 rows, H 1024, V 32000: 3.53 ms materialised, 3.15 accumulated).
+    const bool materialise = budget < 0 && s.ce && s.grad && s.BT > cmax && (s.H >= 2048 || s.chunk_cap > 0);
+    for (const FlChoice& c : all) {
+      const Roundings cr = roundings(s, c);
+      if (cr.dw > rr.dw || cr.dx > rr.dx) continue;
+      if (materialise && (c.vtile || !c.wt || !c.dt || c.dw != kDwDefer)) continue;
+      pick.consider(c);
+    }
+  } else {  // a forced form, or a budget that only a form without X^T fits
+    for (const FlChoice& c : all) pick.consider(c);
   }
-  *out = take ? *take : fast;
+  const FlChoice& c = pick.take();
+  *out = c.vtile ? vt_layout(s, c.C, c.dw) : fl_layout(s, c.C, c.wt, c.dt, c.dw, c.smax, c.part);
+  out->cost = c.cost;
   return HK_OK;
 }
 

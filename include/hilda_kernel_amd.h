@@ -384,7 +384,9 @@ int hk_grpo_loss_fwd(void* dlogits, float* loss_out, float* kl_out, float* clip_
  *     slower; for fp16 inputs such a plan is compared only with the plans
  *     that do not sum dW in the fp16 output over row chunks (there gradients
  *     scaled by 1/n fall in fp16's subnormal range), when one fits
- *     (hk_fused_linear_cross_entropy_plan reports the choice).
+ *     (hk_fused_linear_cross_entropy_plan reports the choice). How often dW
+ *     and dX may be rounded to 16 bits between partial sums is decided with
+ *     rates that stay fixed: a faster kernel never moves a call to fewer bits.
  *   Debugging override (all fused-linear ops, read at every call): the
  *   environment variable HILDA_FL_FORM="<defer|acc|out>,<wt|wmn>,<dt|dmn>"
  *   restricts the plan to that row-chunked form (dW deferred, in an fp32
