@@ -1142,8 +1142,10 @@ struct FlPick {
 // Two models choose. kSumModel, over the forms it prices (tiles of at most 8192
 // columns, X^T in every row-chunked form), makes the choice FlPick describes: it
 // says how often dW and dX may be rounded between partial sums (the reference's
-// own dW is rounded per chunk, fused_linear_cross_entropy.py:161). kModel then
-// chooses in the same way among all forms that round no gradient more often.
+// own dW is rounded per chunk, fused_linear_cross_entropy.py:161) and how many
+// bytes a plan of capped chunks and unlimited budget may take. kModel then
+// chooses in the same way among all forms that round no gradient more often and
+// take no more.
 int fl_plan(const FlShape& s, int64_t budget, FlPlan* out) {
   int f_dw = 0;
   int64_t f_vt = 0;
@@ -1240,14 +1242,19 @@ int fl_plan(const FlShape& s, int64_t budget, FlPlan* out) {
   if (sum.found) {
     const FlChoice& r = sum.take();
     const Roundings rr = roundings(s, r);
-    // Without a limit a FusedLinearCE call of several chunks keeps its documented plan: W^T, every chunk's D^T and
-    // one dW GEMM, with the workspace callers size for it (C5: 39.0 ms; W, D and X read MN-contiguous with an
-    // fp32 dW accumulator 38.4 ms, W alone MN-contiguous 38.2). Small hidden sizes, whose accumulator is cheap,
-    // were and stay the model's choice (16384 rows, H 1024, V 32000: 3.53 ms materialised, 3.15 accumulated).
-    const bool materialise = budget < 0 && s.ce && s.grad && s.BT > cmax && (s.H >= 2048 || s.chunk_cap > 0);
+    // a caller that caps the chunk bounds the workspace by it, also where the budget does not (65536 rows in chunks of
+    // 2048, H 512, V 32000: 11.05 ms with every chunk's D^T in 4.4 GB, 10.45 with an accumulator in 0.23)
+    const size_t bytes = budget < 0 && s.chunk_cap > 0 ? r.total : cap;
+    // Without a limit a FusedLinearCE call of several chunks that kSumModel plans so keeps W^T, every chunk's D^T and
+    // one dW GEMM, with the workspace callers size for it (C5: 39.0 ms; W, D and X read MN-contiguous with an fp32 dW
+    // accumulator 38.4 ms, W alone MN-contiguous 38.2; 4736 rows in chunks of 2048, H 1024, V 128256: 4.37 ms, with an
+    // accumulator 4.47). Small hidden sizes, whose accumulator is cheap, are kModel's choice in chunks of 8192 (16384
+    // rows, H 1024, V 32000: 3.53 ms materialised, 3.15 accumulated).
+    const bool materialise = budget < 0 && s.ce && s.grad && s.BT > cmax && (s.H >= 2048 || s.chunk_cap > 0) &&
+                             !r.vtile && r.wt && r.dt && r.dw == kDwDefer;
     for (const FlChoice& c : all) {
       const Roundings cr = roundings(s, c);
-      if (cr.dw > rr.dw || cr.dx > rr.dx) continue;
+      if (cr.dw > rr.dw || cr.dx > rr.dx || c.total > bytes) continue;
       if (materialise && (c.vtile || !c.wt || !c.dt || c.dw != kDwDefer)) continue;
       pick.consider(c);
     }

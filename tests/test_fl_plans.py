@@ -57,3 +57,21 @@ def test_gradients_are_rounded_no_more_often(op, BT, H, V, budget, dtype, dw, dx
     _, n, mode, *_ = _plan(op, BT, H, V, budget, dtype)
     steps = {2: (n - 1, 0), 4: (0, n - 1)}.get(mode, (0, 0))
     assert steps[0] <= dw and steps[1] <= dx, (mode, n)
+
+
+# (BT, H, V, chunk, most bytes): unlimited budget, capped chunks
+CAPPED = [
+    (51188, 8, 150497, 64, 27740928), (65536, 512, 128256, 2048, 958726656), (65536, 512, 256000, 2048, 1874395648),
+    (16384, 512, 32000, 2048, 267584000), (2176, 1024, 8000, 2048, 136162816), (2176, 5120, 128256, 2048, 928271872),
+    (4736, 1024, 128256, 2048, 2100510208), (896, 4096, 32000, 2048, 173397504),
+    (16384, 4096, 128256, 2048, 6098027008),
+]
+
+
+@needs_lib
+@pytest.mark.parametrize("BT,H,V,chunk,most", CAPPED)
+def test_capped_chunks_bound_the_workspace(BT, H, V, chunk, most):
+    """A caller that caps the chunk also bounds the workspace when the budget does not: no form is forced that keeps
+    every chunk's D^T where an accumulator of a fraction of its size does."""
+    C, *_, total, _ = _plan("ce", BT, H, V, -1, BF16, chunk)
+    assert C <= chunk and total <= most
