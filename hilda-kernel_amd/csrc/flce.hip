@@ -1054,6 +1054,9 @@ bool forced_form(int* dw, bool* wt, bool* dt, int64_t* vt, bool* bad) {
   return true;
 }
 
+// The widest vocabulary tile the dX GEMM's operand panels (256 rows of the tile buffer) can address.
+int64_t widest_tile(int es) { return (int64_t)(gemm::kOobOffset - 1) / (256 * es) / 256 * 256; }
+
 // Default budget floor: below this much chunk memory there is nothing worth
 // saving, and small problems then run in one chunk (or with an fp32 dW
 // accumulator). 40 MiB keeps the reference's tightest memory config
@@ -1216,7 +1219,7 @@ int fl_plan(const FlShape& s, int64_t budget, FlPlan* out) {
   if (s.vt_ok && s.BT > 0 && (forced ? f_vt > 0 : s.chunk_cap <= 0)) {
     // tiles of up to the whole vocabulary (above 8192 columns in steps of 2048): few rows need wide tiles to
     // fill the chip (500 rows of V 128256: a GEMM of 8192 columns has 64 workgroups)
-    const int64_t vmax = (s.V + 255) / 256 * 256;
+    const int64_t vmax = std::min((s.V + 255) / 256 * 256, widest_tile(s.es));
     for (int64_t Vt = vmax; Vt >= 256; Vt = Vt > 8192 ? std::max<int64_t>(8192, (Vt - 1) / 2048 * 2048) : Vt - 256)
       for (int dw : {kDwAcc, kDwOut}) {
         if (forced && (Vt != f_vt || dw != f_dw)) continue;
@@ -1252,7 +1255,10 @@ int fl_plan(const FlShape& s, int64_t budget, FlPlan* out) {
     // rows, H 1024, V 32000: 3.53 ms materialised, 3.15 accumulated).
     const bool materialise = budget < 0 && s.ce && s.grad && s.BT > cmax && (s.H >= 2048 || s.chunk_cap > 0) &&
                              !r.vtile && r.wt && r.dt && r.dw == kDwDefer;
+    // (chunk rows too long for the dX GEMM do not take a call from the tiles)
+    const bool tiles_only = r.vtile && s.grad && pad64(s.V) > widest_tile(s.es);
     for (const FlChoice& c : all) {
+      if (tiles_only && !c.vtile) continue;
       const Roundings cr = roundings(s, c);
       if (cr.dw > rr.dw || cr.dx > rr.dx || c.total > bytes) continue;
       if (materialise && (c.vtile || !c.wt || !c.dt || c.dw != kDwDefer)) continue;

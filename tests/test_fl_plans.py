@@ -75,3 +75,13 @@ def test_capped_chunks_bound_the_workspace(BT, H, V, chunk, most):
     every chunk's D^T where an accumulator of a fraction of its size does."""
     C, *_, total, _ = _plan("ce", BT, H, V, -1, BF16, chunk)
     assert C <= chunk and total <= most
+
+
+@needs_lib
+@pytest.mark.parametrize("BT,H,V,budget", [(8, 64, 20_000_000, M256), (64, 256, 4_300_000, M256),
+                                           (64, 256, 8_000_000, M256), (64, 256, 20_000_000, 1 << 30),
+                                           (8, 64, 100_000_000, 1 << 30), (1024, 64, 100_000_000, 0)])
+def test_tiles_stay_within_a_gemm_panel(BT, H, V, budget):
+    """256 rows of a tile buffer stay below the 2 GiB a GEMM's buffer can address; wider plans fail at launch."""
+    cols, _, mode, *_ = _plan("ce", BT, H, V, budget, BF16)
+    assert mode in (3, 4) and 256 * cols * 2 < 0x7FF00000
