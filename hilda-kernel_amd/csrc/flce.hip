@@ -1044,7 +1044,7 @@ bool forced_form(int* dw, bool* wt, bool* dt, int64_t* vt, bool* bad) {
   if (sa == "vtile") {
     *dw = sb == "acc" ? kDwAcc : sb == "out" ? kDwOut : -1;
     *vt = std::atoll(c);
-    *bad = *dw < 0 || *vt <= 0 || *vt % 256 != 0 || *vt > 8192;
+    *bad = *dw < 0 || *vt <= 0 || *vt % 256 != 0;
     return true;
   }
   *dw = sa == "defer" ? kDwDefer : sa == "acc" ? kDwAcc : sa == "out" ? kDwOut : -1;
@@ -1220,9 +1220,13 @@ int fl_plan(const FlShape& s, int64_t budget, FlPlan* out) {
     // tiles of up to the whole vocabulary (above 8192 columns in steps of 2048): few rows need wide tiles to
     // fill the chip (500 rows of V 128256: a GEMM of 8192 columns has 64 workgroups)
     const int64_t vmax = std::min((s.V + 255) / 256 * 256, widest_tile(s.es));
-    for (int64_t Vt = vmax; Vt >= 256; Vt = Vt > 8192 ? std::max<int64_t>(8192, (Vt - 1) / 2048 * 2048) : Vt - 256)
+    std::vector<int64_t> widths;
+    if (forced) widths.assign(f_vt <= vmax ? 1 : 0, f_vt);
+    for (int64_t Vt = vmax; Vt >= 256 && !forced; Vt = Vt > 8192 ? std::max<int64_t>(8192, (Vt - 1) / 2048 * 2048) : Vt - 256)
+      widths.push_back(Vt);
+    for (int64_t Vt : widths)
       for (int dw : {kDwAcc, kDwOut}) {
-        if (forced && (Vt != f_vt || dw != f_dw)) continue;
+        if (forced && dw != f_dw) continue;
         const FlPlan p = vt_layout(s, Vt, dw);
         if (p.total > cap) continue;
         FlChoice c{Vt, p.ntiles, true, false, false, dw, 1, 0, p.total, vt_cost(s, p, kModel)};
