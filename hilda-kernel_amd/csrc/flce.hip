@@ -1066,9 +1066,13 @@ constexpr size_t kSmallWorkspace = (size_t)40 << 20;
 
 // A plan that sums dW (and dX) in fp32 is taken over a faster one that sums in
 // the 16-bit output unless it is modelled this much slower (by kSumModel, see
-// fl_plan; kModel may only move a call towards fp32). Vocabulary tiles
-// wider than 8192 columns, for few rows: their GEMMs have few workgroups, and
-// beyond 1.3 a call got slower (1024 rows, H 1024, V 50257: 1.26 -> 1.41 ms).
+// fl_plan; kModel may only move a call towards fp32). Vocabulary tiles wider
+// than 8192 columns, for few rows: between 1.3 and 1.5 they took 0.87 to 1.35
+// times as long as the 16-bit sums, 1.15 or more in six of nine calls (1024 rows,
+// H 1024, V 50257: 1.17 -> 1.38 ms; 640 rows, H 2048: 1.79 -> 1.56; 1536 rows,
+// H 4096, V 128256 in 256 MiB: 5.32 -> 7.21); below, they were the faster form
+// (256 rows, H 5120, V 128256: 5.20 -> 4.41; 8576 rows, H 512, V 151936 in 256
+// MiB: 10.4 -> 9.6).
 constexpr double kExactSlack = 1.5, kWideTileSlack = 1.3;
 
 // A candidate plan: what fl_layout (vt_layout) is called with, and its bytes and modelled seconds.
@@ -1254,7 +1258,7 @@ int fl_plan(const FlShape& s, int64_t budget, FlPlan* out) {
     const size_t bytes = budget < 0 && s.chunk_cap > 0 ? r.total : cap;
     // Without a limit a FusedLinearCE call of several chunks that kSumModel plans so keeps W^T, every chunk's D^T and
     // one dW GEMM, with the workspace callers size for it (C5: 39.0 ms; W, D and X read MN-contiguous with an fp32 dW
-    // accumulator 38.4 ms, W alone MN-contiguous 38.2; 4736 rows in chunks of 2048, H 1024, V 128256: 4.37 ms, with an
+    // accumulator 38.2 ms, W alone MN-contiguous 38.2; 4736 rows in chunks of 2048, H 1024, V 128256: 4.37 ms, with an
     // accumulator 4.47). Small hidden sizes, whose accumulator is cheap, are kModel's choice in chunks of 8192 (16384
     // rows, H 1024, V 32000: 3.53 ms materialised, 3.15 accumulated).
     const bool materialise = budget < 0 && s.ce && s.grad && s.BT > cmax && (s.H >= 2048 || s.chunk_cap > 0) &&
@@ -1597,7 +1601,7 @@ namespace {
 // fall back to short chunks, whose dW GEMM re-reads and rewrites the whole
 // weight gradient every chunk: at B 16, L+1 1024, H 4096, V 151936 bf16, 9444
 // live tokens, 100 ms with a 150 MB plan, 31 ms at the floor, 28 ms with no
-// limit.
+// limit (10743 live: 33 and 31).
 size_t weight_pair_bytes(int64_t V, int64_t H, int es) { return 2 * (size_t)V * (size_t)pad8(H) * (size_t)es; }
 
 // Default-budget floor of FusedLinearJSD: what the reference's chunk loop

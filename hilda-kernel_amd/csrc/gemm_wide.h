@@ -6,7 +6,7 @@
 // Bound by the matrix pipes and, in long runs, by the part's power limit. One
 // 256x256 tile a workgroup of 4 waves, one wave a SIMD, each wave 128x128
 // (8x8 16x16x32 MFMAs, 256 accumulators in AGPRs): a wave tile of 128x64 on 8
-// waves, which this replaces, reads a third more LDS bytes per FLOP. K advances
+// waves, which this replaces, reads half as many LDS bytes again per FLOP. K advances
 // 64 a stage through two 64 KiB LDS stages filled by buffer-to-LDS DMA.
 //
 // With one wave a SIMD nothing hides a stall but the order of the instructions,
@@ -37,7 +37,8 @@
 //   B MN-contiguous, read-modify-write 8192x4096x4096  1070 -> 1393-1458
 // A tile's time beyond its K loop (the intercept over K at 8192x32768): 13 us one tile a workgroup -> 7 us, with a
 // read-modify-write epilogue 51 -> 21 us. torch.matmul's best layout at 8192x32000x4096: 1494. In long runs the
-// matrix pipes are 73% busy at 1.9 GHz: the power limit.
+// matrix pipes are 72-80% busy at 1.6-1.8 GHz: the power limit (logits, dX and dW of 16384 rows, H 4096, V 128256: 6.2,
+// 6.2 and 12.1 ms).
 #pragma once
 
 #include "hk_common.h"
@@ -302,7 +303,10 @@ __device__ __forceinline__ void wide_core(unsigned char* __restrict__ a0, unsign
 // with n of the 8 columns from col inside the matrix. An epilogue that reads gets the loads of kBatch chunks in
 // flight, the first batch issued a stage before the tile ends. (Staged through LDS, half a tile at a time, the
 // read-modify-write of a tile took 51 us: four round trips of 8-byte loads with the matrix pipes idle.) One code
-// path for whole and edge tiles: with two, the compiler read all 256 accumulators before their branch and spilled.
+// path for whole and edge tiles: with two, the compiler read all 256 accumulators before their branch and spilled them.
+// Accumulation in a 16-bit output (EpiDw<T, 1>) still spills 24 bytes a lane with B MN-contiguous and 48 with both,
+// beside the transposed reads' bases; the other forms have no scratch. Its GEMM (8192x4096x4096, B MN-contiguous) takes
+// 459 us against 389 without the accumulation, a quarter of the waves' time in waits.
 template <class Epi>
 struct WideOut {
   static constexpr int kBatch = Epi::kReads ? 32 / (int)(sizeof(typename Epi::Prior8) / 4) : 1;  // 32 registers

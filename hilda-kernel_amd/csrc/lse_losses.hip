@@ -65,7 +65,7 @@ struct RowRegs {
   // instead: those that the lane before it also holds count once (mask_tail)
   // and are stored twice, with the same values. (Such rows took one element a
   // lane, in two passes over memory: the GRPO call on [8, 513, 50257] bf16,
-  // two thirds of the rows live, took 325 us and takes 196. Bound by HBM, with
+  // two thirds of the rows live, took 293 us and takes 194. Bound by HBM, with
   // the odd rows' extra cache line a wave.)
   static constexpr int kSpan = BLOCK * VEC;
   __device__ __forceinline__ static Pack<T, VEC> get(const T* p) {
