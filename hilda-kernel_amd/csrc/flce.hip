@@ -1224,10 +1224,11 @@ int fl_plan(const FlShape& s, int64_t budget, FlPlan* out) {
     // tiles of up to the whole vocabulary (above 8192 columns in steps of 2048): few rows need wide tiles to
     // fill the chip (500 rows of V 128256: a GEMM of 8192 columns has 64 workgroups)
     const int64_t vmax = std::min((s.V + 255) / 256 * 256, widest_tile(s.es));
+    auto narrower = [](int64_t Vt) { return Vt > 8192 ? std::max<int64_t>(8192, (Vt - 1) / 2048 * 2048) : Vt - 256; };
     std::vector<int64_t> widths;
     if (forced) widths.assign(f_vt <= vmax ? 1 : 0, f_vt);
-    for (int64_t Vt = vmax; Vt >= 256 && !forced; Vt = Vt > 8192 ? std::max<int64_t>(8192, (Vt - 1) / 2048 * 2048) : Vt - 256)
-      widths.push_back(Vt);
+    else
+      for (int64_t Vt = vmax; Vt >= 256; Vt = narrower(Vt)) widths.push_back(Vt);
     for (int64_t Vt : widths)
       for (int dw : {kDwAcc, kDwOut}) {
         if (forced && dw != f_dw) continue;
